@@ -56,7 +56,10 @@ extern "C" int streams_reactor_batch(int n_s, int nbatch, double *w, double *tgu
                 Thermo{cv_coeff, cp_coeff, trange, nsetcv, indx_cp_l, indx_cp_r}};
   zero_counter_kernel<<<1, 1, 0, st>>>(work);
   const int ncu = device_cus();
-  if ((long)nbatch > (long)ncu * 256)
-    return reactor_dispatch_wide(n_s, indx_cp_l, indx_cp_r, A, ncu, wg_per_cu, st);
-  return reactor_dispatch<false>(n_s, indx_cp_l, indx_cp_r, A, ncu, wg_per_cu, st);
+  if (mixed != 0)
+    return pressure != nullptr ? reactor_group_cp(n_s, indx_cp_l, indx_cp_r, A, ncu, wg_per_cu, st)
+                               : reactor_group_cv(n_s, indx_cp_l, indx_cp_r, A, ncu, wg_per_cu, st);
+  if (indx_cp_r != 4 || (indx_cp_l != 0 && indx_cp_l != -2)) return STREAMS_E_OPTION;
+  if ((long)nbatch > (long)ncu * 256) return reactor_dispatch_wide(n_s, A, ncu, wg_per_cu, st);
+  return reactor_dispatch<false>(n_s, A, ncu, wg_per_cu, st);
 }
