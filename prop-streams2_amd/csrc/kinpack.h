@@ -95,6 +95,68 @@ struct RefSpecies<NS, NS> {
   __device__ static inline void accumulate(kdouble *, kint *, int, int, double, const double *, double *) {}
 };
 
+// Rate of progress of one reaction in the forms of REF = false.  The record and conc(s) are
+// read through the caller's pointers: wave-uniform scalar loads when every lane walks the same
+// reaction, vector loads when each lane takes its own.  kc points at K_c's table row.  pick(s)
+// is conc(s) where s comes from the record (a register array would be indexed dynamically).
+template <int NS, class RD, class RI, class Conc, class Pick>
+__device__ inline double reaction_progress(RD R, RI I, const double *kc, double tt, double lnT, double Rtti, double dtt,
+                                           const Conc &conc, const Pick &pick) {
+  constexpr double LN10 = 2.302585092994045684;
+  constexpr double ILN10 = 0.434294481903251827651;
+  const int ty = I[KI_TY];
+  double kf, tbv = 1.0;
+  if (ty <= 1) {
+    kf = R[KD_A];
+    if (I[KI_ARR]) kf = kf * exp(R[KD_A + 1] * lnT - R[KD_A + 2] * Rtti);
+    if (ty == 1) {
+      tbv = 0.0;
+#pragma unroll
+      for (int s = 0; s < NS; ++s) tbv = tbv + R[KD_TB + s] * conc(s);
+    }
+  } else {
+    const double k0 = R[KD_A] * exp(R[KD_A + 1] * lnT - R[KD_A + 2] * Rtti);
+    const double kinf = R[KD_AINF] * exp(R[KD_AINF + 1] * lnT - R[KD_AINF + 2] * Rtti);
+    double tb = 0.0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) tb = tb + R[KD_TB + s] * conc(s);
+    const double rpres = k0 * tb / kinf;
+    if (ty == 2) {
+      kf = kinf * (rpres / (1.0 + rpres));
+    } else if (ty == 3) {
+      if (rpres < 1e-30) {
+        kf = k0 * tb;
+      } else {
+        double fcent = (1.0 - R[KD_FC]) * exp(-tt / R[KD_FC + 1]) + R[KD_FC] * exp(-tt / R[KD_FC + 2]);
+        if (I[KI_T2]) fcent = fcent + exp(-R[KD_FC + 3] / tt);
+        fcent = log(fcent) * ILN10;
+        const double coff = -0.4 - 0.67 * fcent;
+        const double noff = 0.75 - 1.27 * fcent;
+        const double lr10 = log(rpres) * ILN10;
+        const double fo = (lr10 + coff) / (noff - 0.14 * (lr10 + coff));
+        kf = kinf * (rpres / (1.0 + rpres)) * exp(LN10 * (fcent / (1.0 + fo * fo)));
+      }
+    } else {
+      const double l10 = log(rpres) * ILN10;
+      const double xoff = 1.0 / (1.0 + l10 * l10);
+      const double sri = R[KD_FC] * exp(-R[KD_FC + 1] / tt) + exp(-tt / R[KD_FC + 2]);
+      const double foff = R[KD_FC + 3] * exp(xoff * log(sri)) * exp(R[KD_FC + 4] * lnT);
+      kf = kinf * (rpres / (1.0 + rpres)) * foff;
+    }
+  }
+  double kb = 0.0;
+  if (I[KI_REV] == 1) kb = kf / (kc[0] + (kc[1] - kc[0]) * dtt);
+  double q1 = 1.0, q2 = 1.0;
+  const int nre = I[KI_NRE], npr = I[KI_NPR];
+#pragma unroll
+  for (int e = 0; e < KSIDE; ++e)
+    if (e < nre) q1 = q1 * conc_power(pick(I[KI_RE + e]), R[KD_REX + e]);
+#pragma unroll
+  for (int e = 0; e < KSIDE; ++e)
+    if (e < npr) q2 = q2 * conc_power(pick(I[KI_PR + e]), R[KD_PEX + e]);
+  return tbv * (kf * q1 - kb * q2);
+}
+
 // Species source -omega_s W_s accumulated into acc[0..NS) for one cell at temperature tt
 // with molar concentrations conc (compute_chemistry_cuf's reaction loop,
 // kernels_gpu.F90:9551-9649).
@@ -107,12 +169,10 @@ struct RefSpecies<NS, NS> {
 //    with the b = 0 and Ea = 0 cases skipped, log10, pow(10, .), pow for exponents other
 //    than 1, products over the species in ascending order, acc -= ((p - r) q) W_s with
 //    mw = W_s.
-template <int NS, bool REF = false>
-__device__ inline void chemistry_source_packed(const KinPacked &K, double tt, const double *conc, double *acc,
-                                               const double *mw = nullptr) {
+template <int NS, bool REF, class Pick>
+__device__ inline void chemistry_source_from(const KinPacked &K, double tt, const double *conc, double *acc,
+                                             const double *mw, const Pick &pick) {
   static_assert(NS <= KTB, "third-body efficiencies of a record hold at most KTB species");
-  constexpr double LN10 = 2.302585092994045684;
-  constexpr double ILN10 = 0.434294481903251827651;
   const double Rtti = 1.0 / (K.r_univ * tt);
   const double lnT = log(tt);
   int itt = (int)((tt - K.t_min_tab) / K.dt_tab) + 1;
@@ -124,9 +184,10 @@ __device__ inline void chemistry_source_packed(const KinPacked &K, double tt, co
   for (int lr = 0; lr < K.nr; ++lr) {
     kdouble *R = (kdouble *)K.pack + KREC * lr;
     kint *I = (kint *)R;
-    const int ty = I[KI_TY];
-    double kf, tbv = 1.0;
+    const double *kp = K.kc_tab + (itt - 1) + ntab * lr;
     if (REF) {
+      const int ty = I[KI_TY];
+      double kf, tbv = 1.0;
       if (ty <= 1) {
         kf = R[KD_A];
         if (R[KD_A + 1] != 0.0) kf = kf * pow(tt, R[KD_A + 1]);
@@ -167,67 +228,25 @@ __device__ inline void chemistry_source_packed(const KinPacked &K, double tt, co
           kf = kinf * (rpres / (1.0 + rpres)) * foff;
         }
       }
-    } else if (ty <= 1) {
-      kf = R[KD_A];
-      if (I[KI_ARR]) kf = kf * exp(R[KD_A + 1] * lnT - R[KD_A + 2] * Rtti);
-      if (ty == 1) {
-        tbv = 0.0;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) tbv = tbv + R[KD_TB + s] * conc[s];
-      }
-    } else {
-      const double k0 = R[KD_A] * exp(R[KD_A + 1] * lnT - R[KD_A + 2] * Rtti);
-      const double kinf = R[KD_AINF] * exp(R[KD_AINF + 1] * lnT - R[KD_AINF + 2] * Rtti);
-      double tb = 0.0;
-#pragma unroll
-      for (int s = 0; s < NS; ++s) tb = tb + R[KD_TB + s] * conc[s];
-      const double rpres = k0 * tb / kinf;
-      if (ty == 2) {
-        kf = kinf * (rpres / (1.0 + rpres));
-      } else if (ty == 3) {
-        if (rpres < 1e-30) {
-          kf = k0 * tb;
-        } else {
-          double fcent = (1.0 - R[KD_FC]) * exp(-tt / R[KD_FC + 1]) + R[KD_FC] * exp(-tt / R[KD_FC + 2]);
-          if (I[KI_T2]) fcent = fcent + exp(-R[KD_FC + 3] / tt);
-          fcent = log(fcent) * ILN10;
-          const double coff = -0.4 - 0.67 * fcent;
-          const double noff = 0.75 - 1.27 * fcent;
-          const double lr10 = log(rpres) * ILN10;
-          const double fo = (lr10 + coff) / (noff - 0.14 * (lr10 + coff));
-          kf = kinf * (rpres / (1.0 + rpres)) * exp(LN10 * (fcent / (1.0 + fo * fo)));
-        }
-      } else {
-        const double l10 = log(rpres) * ILN10;
-        const double xoff = 1.0 / (1.0 + l10 * l10);
-        const double sri = R[KD_FC] * exp(-R[KD_FC + 1] / tt) + exp(-tt / R[KD_FC + 2]);
-        const double foff = R[KD_FC + 3] * exp(xoff * log(sri)) * exp(R[KD_FC + 4] * lnT);
-        kf = kinf * (rpres / (1.0 + rpres)) * foff;
-      }
-    }
-    double kb = 0.0;
-    if (I[KI_REV] == 1) {
-      const double *kp = K.kc_tab + (itt - 1) + ntab * lr;
-      kb = kf / (kp[0] + (kp[1] - kp[0]) * dtt);
-    }
-    double q1 = 1.0, q2 = 1.0;
-    const int nre = I[KI_NRE], npr = I[KI_NPR];
-    if (REF) {
+      double kb = 0.0;
+      if (I[KI_REV] == 1) kb = kf / (kp[0] + (kp[1] - kp[0]) * dtt);
+      double q1 = 1.0, q2 = 1.0;
+      const int nre = I[KI_NRE], npr = I[KI_NPR];
       RefSpecies<0, NS>::products(R, I, nre, npr, conc, q1, q2);
       const double q = tbv * (kf * q1 - kb * q2);
       RefSpecies<0, NS>::accumulate(R, I, nre, npr, q, mw, acc);
     } else {
-#pragma unroll
-      for (int e = 0; e < KSIDE; ++e)
-        if (e < nre) q1 = q1 * conc_power(conc[I[KI_RE + e]], R[KD_REX + e]);
-#pragma unroll
-      for (int e = 0; e < KSIDE; ++e)
-        if (e < npr) q2 = q2 * conc_power(conc[I[KI_PR + e]], R[KD_PEX + e]);
-      const double q = tbv * (kf * q1 - kb * q2);
+      const double q = reaction_progress<NS>(R, I, kp, tt, lnT, Rtti, dtt, [&](int s) { return conc[s]; }, pick);
 #pragma unroll
       for (int s = 0; s < NS; ++s) acc[s] = acc[s] - q * R[KD_NET + s];
     }
   }
+}
+
+template <int NS, bool REF = false>
+__device__ inline void chemistry_source_packed(const KinPacked &K, double tt, const double *conc, double *acc,
+                                               const double *mw = nullptr) {
+  chemistry_source_from<NS, REF>(K, tt, conc, acc, mw, [&](int s) { return conc[s]; });
 }
 
 }  // namespace streams

@@ -19,13 +19,15 @@ struct RosRhsPacked {
   const ThermoLds &TL;
   const double *mw;
   double tol_iter_nr;
-  // the temperature of state wv (species not negative), from the guess tg
-  __device__ inline void temperature(const double *wv, double &tg) const {
+  // the temperature of state wv (species not negative), from the guess tg; density, the
+  // factor ri that makes mass fractions of the state, and scale
+  __device__ inline void prepare(const double *wv, double &tg, double &rho, double &ri, double &scale) const {
     double yy[NS];
-    double rho = wv[0];
+    rho = wv[0];
 #pragma unroll
     for (int s = 1; s < NS; ++s) rho = rho + wv[s];
-    const double ri = 1.0 / rho;
+    ri = 1.0 / rho;
+    scale = 1.0;
 #pragma unroll
     for (int s = 0; s < NS; ++s) yy[s] = wv[s] * ri;
     const double uu = wv[NS] * ri, vv = wv[NS + 1] * ri, ww = wv[NS + 2] * ri;
@@ -34,8 +36,9 @@ struct RosRhsPacked {
     int nrange[NS];
     tg = temperature_from_e_lds<NS, LO>(ee, tg, TL, tol_iter_nr, yy, nrange);
   }
-  // fix: tg is the state's temperature already
-  __device__ inline double operator()(double *wv, double &tg, double *rhs, bool fix) const {
+  // fix: tg is the state's temperature already; the lane's concentrations are also kept in
+  // cbuf (species stride cst) for the products that a record's species indices pick
+  __device__ inline double operator()(double *wv, double &tg, double *rhs, bool fix, double *cbuf, int cst) const {
     double yy[NS], conc[NS], acc[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) wv[s] = wv[s] > 0.0 ? wv[s] : 0.0;
@@ -48,6 +51,7 @@ struct RosRhsPacked {
       yy[s] = wv[s] * ri;
       conc[s] = rho * yy[s] / mw[s];
       acc[s] = 0.0;
+      cbuf[s * cst] = conc[s];
     }
     const double uu = wv[NS] * ri, vv = wv[NS + 1] * ri, ww = wv[NS + 2] * ri;
     const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
@@ -55,7 +59,7 @@ struct RosRhsPacked {
     int nrange[NS];
     const double tt = temperature_from_e_lds<NS, LO>(ee, tg, TL, tol_iter_nr, yy, nrange);
     tg = fix ? tg : tt;
-    chemistry_source_packed<NS>(K, tg, conc, acc);
+    chemistry_source_from<NS, false>(K, tg, conc, acc, nullptr, [&](int s) { return cbuf[s * cst]; });
 #pragma unroll
     for (int s = 0; s < NS; ++s) rhs[s] = -acc[s];
     return 1.0;
@@ -72,18 +76,24 @@ struct RosRhsPressure {
   const ThermoLds &TL;
   const double *mw, *rgas;
   double pres, tol_iter_nr;
-  __device__ inline void temperature(const double *wv, double &tg) const {
+  __device__ inline void prepare(const double *wv, double &tg, double &rho, double &yi, double &scale) const {
     double yy[NS];
     double ysum = wv[0];
 #pragma unroll
     for (int s = 1; s < NS; ++s) ysum = ysum + wv[s];
-    const double yi = 1.0 / ysum;
+    yi = 1.0 / ysum;
+    double rmix = 0.0;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) yy[s] = wv[s] * yi;
+    for (int s = 0; s < NS; ++s) {
+      yy[s] = wv[s] * yi;
+      rmix = rmix + rgas[s] * yy[s];
+    }
     int nrange[NS];
     tg = temperature_newton_lds<NS, LO>(wv[NS + 3], tg, TL, TL.cp, TL.cph, tol_iter_nr, yy, nrange);
+    rho = pres / (rmix * tg);
+    scale = 1.0 / rho;
   }
-  __device__ inline double operator()(double *wv, double &tg, double *rhs, bool fix) const {
+  __device__ inline double operator()(double *wv, double &tg, double *rhs, bool fix, double *cbuf, int cst) const {
     double yy[NS], conc[NS], acc[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) wv[s] = wv[s] > 0.0 ? wv[s] : 0.0;
@@ -105,8 +115,9 @@ struct RosRhsPressure {
     for (int s = 0; s < NS; ++s) {
       conc[s] = rho * yy[s] / mw[s];
       acc[s] = 0.0;
+      cbuf[s * cst] = conc[s];
     }
-    chemistry_source_packed<NS>(K, tg, conc, acc);
+    chemistry_source_from<NS, false>(K, tg, conc, acc, nullptr, [&](int s) { return cbuf[s * cst]; });
 #pragma unroll
     for (int s = 0; s < NS; ++s) rhs[s] = -acc[s];
     return 1.0 / rho;

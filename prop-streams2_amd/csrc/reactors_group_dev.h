@@ -140,8 +140,48 @@ __device__ inline double row_solve(const double *jrow, const LU *a, int l, int p
   }
 }
 
+// Orders LDS accesses of a wave's lanes: what was written before it is read after it.
+__device__ inline void row_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// chemistry_source_packed of one state with a reaction per lane: c is species l's
+// concentration, the result component l of the source.  The rates of 16 reactions meet in
+// LDS and lane l subtracts them in ascending order.
+template <int NS>
+__device__ inline double row_source(const KinPacked &K, double tt, double c, double *cl, double *ql, int l) {
+  const double Rtti = 1.0 / (K.r_univ * tt);
+  const double lnT = log(tt);
+  int itt = (int)((tt - K.t_min_tab) / K.dt_tab) + 1;
+  itt = itt < 1 ? 1 : itt;
+  itt = itt > K.num_t_tab ? K.num_t_tab : itt;
+  const double ttleft = (itt - 1) * K.dt_tab + K.t_min_tab;
+  const double dtt = (tt - ttleft) / K.dt_tab;
+  const long ntab = (long)K.num_t_tab + 1;
+  double acc = 0.0;
+  cl[l] = c;
+  for (int r0 = 0; r0 < K.nr; r0 += GROW) {
+    const int r = r0 + l;
+    row_sync();
+    if (r < K.nr) {
+      const double *R = K.pack + KREC * r;
+      ql[l] = reaction_progress<NS>(R, (const int *)R, K.kc_tab + (itt - 1) + ntab * r, tt, lnT, Rtti, dtt,
+                                    [&](int s) { return cl[s]; }, [&](int s) { return cl[s]; });
+    }
+    row_sync();
+    const int n = K.nr - r0 < GROW ? K.nr - r0 : GROW;
+    const double *net = K.pack + KREC * r0 + KD_NET + l;
+#pragma unroll 4
+    for (int k = 0; k < n; ++k) acc = acc - ql[k] * net[KREC * k];
+  }
+  row_sync();
+  return acc;
+}
+
 template <int NS, int LO, int MODE, bool CP>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) reactor_group_kernel(ReactorArgs A) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 9 ? 3 : 2))) reactor_group_kernel(ReactorArgs A) {
   using LU = std::conditional_t<MODE == 1, float, double>;
   static_assert(NS < GROW, "a row holds the N_S columns and the base state");
   constexpr int WHICH = CP ? (TH_CP | TH_CPH) : (TH_CV | TH_CVH);
@@ -153,10 +193,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) r
   constexpr double e1 = 17.0 / 54.0, e2 = 7.0 / 36.0, e3 = 0.0, e4 = 125.0 / 108.0;
   __shared__ double tlds[thermo_lds_doubles<NS>(WHICH)];
   __shared__ double jbuf[256 / GROW][NS * (GROW + 1)];
+  __shared__ double cbuf[256 / GROW][2 * GROW];
+  __shared__ double lane_conc[NS * 256];
   const ThermoLds TL = thermo_stage<NS, LO>(A.th, tlds, WHICH);
   __syncthreads();
   const int l = threadIdx.x % GROW;
   double *J = jbuf[threadIdx.x / GROW];
+  double *cl = cbuf[threadIdx.x / GROW], *ql = cl + GROW;
+  const double mwl = A.mw[l < NS ? l : 0];
   const long nb = A.nbatch;
   const double itol = 1.0 / A.tol;
   bool active = false, fresh = true;
@@ -165,23 +209,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) r
   double mom[4] = {0.0, 0.0, 0.0, 0.0};            // momentum and energy (enthalpy): constant
   double tg = 0.0, t0 = 0.0, time = 0.0, dt = 0.0, time_end = 0.0, pres = 0.0;
   int iter = 0, jtry = 0, finish = 0, nacc = 0, nrej = 0;
-  // right-hand side at this lane's state; fix: keep the temperature tfix
-  auto rhs_all = [&](double *wv, double &t, double *out, bool fix) {
-    if constexpr (CP) {
-      const RosRhsPressure<NS, LO> f{A.K, TL, A.mw, A.rgas, pres, A.tol_iter_nr};
-      return f(wv, t, out, fix);
-    } else {
-      const RosRhsPacked<NS, LO> f{A.K, TL, A.mw, A.tol_iter_nr};
-      return f(wv, t, out, fix);
-    }
+  auto rhs_fn = [&]() {
+    if constexpr (CP) return RosRhsPressure<NS, LO>{A.K, TL, A.mw, A.rgas, pres, A.tol_iter_nr};
+    else return RosRhsPacked<NS, LO>{A.K, TL, A.mw, A.tol_iter_nr};
   };
   // stage state v (component l): component l of its right-hand side, unscaled, and the scale
   auto rhs_stage = [&](double v, double &scale) {
-    double wv[NS + 4], out[NS];
+    double wv[NS + 4], rho, ri;
+    v = v > 0.0 ? v : 0.0;
     static_for<0, NS>([&](auto S) { wv[S] = row_bcast<S>(v); });
     static_for<0, 4>([&](auto S) { wv[NS + S] = mom[S]; });
-    scale = rhs_all(wv, tg, out, false);
-    return own<NS>(out, l);
+    rhs_fn().prepare(wv, tg, rho, ri, scale);
+    return -row_source<NS>(A.K, tg, rho * (v * ri) / mwl, cl, ql, l);
   };
   // scale * r + x
   auto scaled_plus = [&](double r, double scale, double x) { return CP ? fma(r, scale, x) : r + x; };
@@ -222,21 +261,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) r
       static_for<0, NS>([&](auto S) { wv[S] = row_bcast<S>(w); });
       static_for<0, 4>([&](auto S) { wv[NS + S] = mom[S]; });
       const double h = w * 1.0e-06 + 1.0e-14;
+      double rho, ri, sc;
+      rhs_fn().prepare(wv, tg, rho, ri, sc);
       double tj = tg;
-      if constexpr (CP) RosRhsPressure<NS, LO>{A.K, TL, A.mw, A.rgas, pres, A.tol_iter_nr}.temperature(wv, tj);
-      else RosRhsPacked<NS, LO>{A.K, TL, A.mw, A.tol_iter_nr}.temperature(wv, tj);
-      tg = tj;
       static_for<0, NS>([&](auto S) { wv[S] = l == S ? w + h : wv[S]; });
-      const double scale = rhs_all(wv, tj, rp, l >= NS);
+      const double scale = rhs_fn()(wv, tj, rp, l >= NS, lane_conc + threadIdx.x, 256);
       static_for<0, NS>([&](auto M) {
         const double base = row_bcast<NS>(CP ? rp[M] * scale : rp[M]);
         if (l == M) rhs_sav = base;
         const double jm = (CP ? fma(rp[M], scale, -base) : rp[M] - base) / h;
         if (l < NS) J[M + (GROW + 1) * l] = jm;
       });
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      row_sync();
       wsav = w;
       jtry = 1;
       fresh = false;
