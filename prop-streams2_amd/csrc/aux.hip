@@ -30,19 +30,17 @@ struct AuxTables {
 // which overwrites it with the conductivity.
 template <int NS, int LO, bool LES = false>
 __global__ void __launch_bounds__(256) eval_aux_kernel(Box b, int istart, int jstart, int kstart,
-                                                       int ni, int nj, long npts, double *__restrict__ w,
+                                                       unsigned ni, unsigned nj, unsigned npts, double *__restrict__ w,
                                                        double *__restrict__ w_aux, Thermo th,
                                                        AuxTables tb, double tol_iter_nr) {
   using X = Idx<NS>;
   __shared__ double tlds[thermo_lds_doubles<NS>(TH_CP | TH_CV | TH_CVH)];
   const ThermoLds TL = thermo_stage<NS, LO>(th, tlds, TH_CP | TH_CV | TH_CVH);
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  __syncthreads();
+  const unsigned t = blockIdx.x * 256u + threadIdx.x;
   if (t >= npts) return;
-  int i = istart + (int)(t % ni);
-  long r = t / ni;
-  int j = jstart + (int)(r % nj);
-  int k = kstart + (int)(r / nj);
-  const long pt = b.p(i, j, k), ps = b.pstride();
+  const unsigned r = t / ni;
+  const long pt = b.p(istart + (int)(t % ni), jstart + (int)(r % nj), kstart + (int)(r / nj)), ps = b.pstride();
 
   double yy[NS];
   double rho = 0.0, uu, vv, ww;
@@ -125,8 +123,8 @@ __global__ void __launch_bounds__(256) eval_aux_kernel(Box b, int istart, int js
 // LES = true adds the eddy viscosity mu_sgs (J_LES1) as eval_aux_les_cuf does: mu + mu_sgs,
 // k + mu_sgs c_p / Pr_sgs (c_p left in J_K_COND by the thermo kernel), rho D_s + mu_sgs / Sc_sgs.
 template <int NS, bool LES = false>
-__global__ void __launch_bounds__(256) eval_transport_kernel(Box b, int istart, int jstart, int kstart, int ni,
-                                                             int nj, long npts, double *__restrict__ w_aux,
+__global__ void __launch_bounds__(256) eval_transport_kernel(Box b, int istart, int jstart, int kstart, unsigned ni,
+                                                             unsigned nj, unsigned npts, double *__restrict__ w_aux,
                                                              AuxTables tb, double les_pr = 0.0,
                                                              double les_sc = 0.0) {
   using X = Idx<NS>;
@@ -138,13 +136,10 @@ __global__ void __launch_bounds__(256) eval_transport_kernel(Box b, int istart, 
     c_pow[q] = pow(tb.mw[m] * tb.mwinv[l], 0.25);
   }
   __syncthreads();
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const unsigned t = blockIdx.x * 256u + threadIdx.x;
   if (t >= npts) return;
-  int i = istart + (int)(t % ni);
-  long r = t / ni;
-  int j = jstart + (int)(r % nj);
-  int k = kstart + (int)(r / nj);
-  const long pt = b.p(i, j, k), ps = b.pstride();
+  const unsigned r = t / ni;
+  const long pt = b.p(istart + (int)(t % ni), jstart + (int)(r % nj), kstart + (int)(r / nj)), ps = b.pstride();
   double yy[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) yy[s] = w_aux[pt + ps * s];
@@ -166,9 +161,8 @@ __global__ void __launch_bounds__(256) eval_transport_kernel(Box b, int istart, 
   double k1 = 0.0, k2 = 0.0;
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    const double *lp = tb.lambda + (itt - 1) + nt * s;
-    double l0 = lp[0], l1 = lp[1];
-    double klsp = l0 + (l1 - l0) * dtt;
+    const DoublePair lp = load_pair(tb.lambda + (itt - 1) + nt * s);
+    double klsp = lp.a + (lp.b - lp.a) * dtt;
     const double xs = yy[s] * mwmixt * tb.mwinv[s];
     k1 = k1 + xs * klsp;
     k2 = k2 + xs * rcp_nr(klsp);
@@ -178,9 +172,8 @@ __global__ void __launch_bounds__(256) eval_transport_kernel(Box b, int istart, 
   double mus[NS], smu[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    const double *vp = tb.visc + (itt - 1) + nt * s;
-    double v0 = vp[0], v1 = vp[1];
-    mus[s] = v0 + (v1 - v0) * dtt;
+    const DoublePair vp = load_pair(tb.visc + (itt - 1) + nt * s);
+    mus[s] = vp.a + (vp.b - vp.a) * dtt;
     smu[s] = sqrt(mus[s]);
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -225,9 +218,8 @@ __global__ void __launch_bounds__(256) eval_transport_kernel(Box b, int istart, 
 #pragma unroll
     for (int m = 0; m < NS; ++m) {
       if (m != l) {
-        const double *dp = tb.diffbin + (itt - 1) + nt * (l + NS * m);
-        double d0 = dp[0], d1 = dp[1];
-        double dij = d0 + (d1 - d0) * dtt;
+        const DoublePair dp = load_pair(tb.diffbin + (itt - 1) + nt * (l + NS * m));
+        double dij = dp.a + (dp.b - dp.a) * dtt;
         dden = dden + xs[m] * rcp_nr(dij);
       }
     }
@@ -325,6 +317,7 @@ extern "C" int streams_eval_aux(int n_s, int nx, int ny, int nz, int ng, int nv,
                dt_tab, p0, r_univ, n_eoi, aw_eoi, beta0, coeff_eoi, nainsp};
   int ni = iend - istart + 1, nj = jend - jstart + 1, nk = kend - kstart + 1;
   long npts = (long)ni * nj * nk;
+  if (npts > 0xffffff00l) return STREAMS_E_DIMS;      // the kernels index points with 32 bits
   STREAMS_DISPATCH_NS(n_s, STREAMS_DISPATCH_NASA(indx_cp_l, indx_cp_r,
                                (eval_aux_kernel<NS, LO><<<blocks_for(npts, 256), 256, 0, as_stream(stream)>>>(
                                    b, istart, jstart, kstart, ni, nj, npts, w, w_aux, th, tb, tol_iter_nr),
@@ -381,6 +374,7 @@ extern "C" int streams_eval_aux_les(int n_s, int nx, int ny, int nz, int ng, int
                dt_tab, p0, r_univ, 1, nullptr, nullptr, nullptr, nullptr};
   const int ni = nx + 2 * ng, nj = ny + 2 * ng;
   const long npts = b.pstride();
+  if (npts > 0xffffff00l) return STREAMS_E_DIMS;
   STREAMS_DISPATCH_NS(n_s, STREAMS_DISPATCH_NASA(indx_cp_l, indx_cp_r,
                                (eval_aux_kernel<NS, LO, true><<<blocks_for(npts, 256), 256, 0, as_stream(stream)>>>(
                                    b, 1 - ng, 1 - ng, 1 - ng, ni, nj, npts, w, w_aux, th, tb, tol_iter_nr),

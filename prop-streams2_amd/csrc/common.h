@@ -46,6 +46,16 @@ __device__ inline double rcp_nr(double d) {
   return fma(r, e, r);
 }
 
+// p[0] and p[1] in one 16-byte load (8-byte aligned): a wave's load instruction costs 16-17
+// cycles of its CU's L1 whether a lane takes 8 or 16 bytes, so a table's two neighbours are
+// read together.
+struct DoublePair { double a, b; };
+__device__ inline DoublePair load_pair(const double *p) {
+  DoublePair v;
+  __builtin_memcpy(&v, p, sizeof(v));
+  return v;
+}
+
 // index of variables (index_define.h), 1-based as in the reference
 template <int NS> struct Idx {
   static constexpr int I_U = NS + 1, I_V = NS + 2, I_W = NS + 3, I_E = NS + 4;

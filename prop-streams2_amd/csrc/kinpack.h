@@ -145,7 +145,10 @@ __device__ inline double reaction_progress(RD R, RI I, const double *kc, double 
     }
   }
   double kb = 0.0;
-  if (I[KI_REV] == 1) kb = kf / (kc[0] + (kc[1] - kc[0]) * dtt);
+  if (I[KI_REV] == 1) {
+    const DoublePair k = load_pair(kc);
+    kb = kf / (k.a + (k.b - k.a) * dtt);
+  }
   double q1 = 1.0, q2 = 1.0;
   const int nre = I[KI_NRE], npr = I[KI_NPR];
 #pragma unroll
