@@ -440,6 +440,23 @@ int streams_rhs_finish_next(int n_s, int nx, int ny, int nz, int ng, int nv_aux,
                             int num_t_tab, double t_min_tab, double dt_tab, double r_univ,
                             double gamdt, double rhodt_next, const int *fluid_mask, void *stream);
 
+/* The three sweeps (visc=1) and the tail (reduced=1) of one substep in one pass over the cells,
+ * for a 3-D box in which every face takes the KEEP flux of one order: nkeep = 0, no face
+ * shocked, no entry of ep_ord_change set, no forced-zero face, lmax_base 3 or 4 =
+ * visc_order/2, NASA7 tables (indx_cp_l = 0), a padded plane of less than 2^29 points.
+ * init=1 also performs init_flux_cuf (fln = -rhodt*fl_old), init=2 takes fln as a folded
+ * substep left it; fold=1 leaves -rhodt_next*fl in fln and does not store fl, as
+ * streams_rhs_finish_next. */
+int streams_rhs_cells(int n_s, int nx, int ny, int nz, int ng, int nv_aux, int lmax_base,
+                      double *w, const double *w_aux, double *fl, double *fln,
+                      const double *coeff_deriv1, const double *dcsidx, const double *detady,
+                      const double *dzitdz, const double *x, const double *y, const double *z,
+                      const double *cp_coeff, int nsetcv, const double *trange, int indx_cp_l,
+                      int indx_cp_r, double r_univ, int chem, int nreactions, const double *mw,
+                      const double *kin_pack, const double *kc_tab, int num_t_tab,
+                      double t_min_tab, double dt_tab, int init, double rhodt, double gamdt,
+                      int fold, double rhodt_next, const int *fluid_mask, void *stream);
+
 /* ---- batched chemistry ---------------------------------------------------------------- */
 /* nbatch independent reactors, each integrated like one cell of rosenbrock_kernel
  * (kernels_gpu.F90:8928-9193, launched by rosenbrock, multideal_gpu.F90:694-767) from t = 0

@@ -7,22 +7,9 @@
 // w_aux as written by eval_aux in the same substep: w is unchanged since then, so rho and
 // Y are the identical numbers compute_chemistry_cuf recomputes; its extra Newton iteration
 // moves T by less than the 1e-12 K stopping tolerance.
-#include "kinpack.h"
+#include "finish.h"
 
 namespace streams {
-
-struct FinishArgs {
-  const double *cd1, *dcsidx, *detady, *dzitdz;
-  const int *mask;
-  const double *mw;
-  KinPacked K;
-  int lmax, reduced, chem;
-  double gamdt;
-  // fold = 1: the next substep's init_flux is done here (fln = -rhodt_next * fl, written in
-  // place of fl, which then needs no store: the next x sweep overwrites it with init = 2)
-  int fold;
-  double rhodt_next;
-};
 
 // One interior cell per thread, i fastest, so that every access of a wave is a coalesced
 // 512-byte segment of one variable plane.  The species equations (chemistry, then their RK
@@ -169,6 +156,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) f
     }
     if (fluid) w[pt + ps * (NS + m)] = w[pt + ps * (NS + m)] + fn;
   }
+}
+
+int finish_species_launch(int n_s, const Box &b, double *w, const double *w_aux, double *fl, double *fln,
+                          const FinishArgs &F, hipStream_t st) {
+  STREAMS_DISPATCH_NS(n_s, (finish_species_kernel<NS><<<blocks_for(b.fstride(), 256), 256, 0, st>>>(b, w, w_aux, fl, fln, F)));
+  return hip_status();
 }
 
 }  // namespace streams

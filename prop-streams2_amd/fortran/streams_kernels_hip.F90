@@ -1029,6 +1029,52 @@ module streams_kernels_hip
       type(c_ptr), value :: fluid_mask
       type(c_ptr), value :: stream
     end function streams_rhs_finish_next
+    integer(c_int) function streams_rhs_cells(n_s, nx, ny, nz, ng, nv_aux, lmax_base, w, w_aux, fl, &
+        fln, coeff_deriv1, dcsidx, detady, dzitdz, x, y, z, cp_coeff, nsetcv, trange, indx_cp_l, &
+        indx_cp_r, r_univ, chem, nreactions, mw, kin_pack, kc_tab, num_t_tab, t_min_tab, dt_tab, &
+        init, rhodt, gamdt, fold, rhodt_next, fluid_mask, stream) &
+        bind(C, name="streams_rhs_cells")
+      import :: c_int, c_double, c_ptr
+      integer(c_int), value :: n_s
+      integer(c_int), value :: nx
+      integer(c_int), value :: ny
+      integer(c_int), value :: nz
+      integer(c_int), value :: ng
+      integer(c_int), value :: nv_aux
+      integer(c_int), value :: lmax_base
+      type(c_ptr), value :: w
+      type(c_ptr), value :: w_aux
+      type(c_ptr), value :: fl
+      type(c_ptr), value :: fln
+      type(c_ptr), value :: coeff_deriv1
+      type(c_ptr), value :: dcsidx
+      type(c_ptr), value :: detady
+      type(c_ptr), value :: dzitdz
+      type(c_ptr), value :: x
+      type(c_ptr), value :: y
+      type(c_ptr), value :: z
+      type(c_ptr), value :: cp_coeff
+      integer(c_int), value :: nsetcv
+      type(c_ptr), value :: trange
+      integer(c_int), value :: indx_cp_l
+      integer(c_int), value :: indx_cp_r
+      real(c_double), value :: r_univ
+      integer(c_int), value :: chem
+      integer(c_int), value :: nreactions
+      type(c_ptr), value :: mw
+      type(c_ptr), value :: kin_pack
+      type(c_ptr), value :: kc_tab
+      integer(c_int), value :: num_t_tab
+      real(c_double), value :: t_min_tab
+      real(c_double), value :: dt_tab
+      integer(c_int), value :: init
+      real(c_double), value :: rhodt
+      real(c_double), value :: gamdt
+      integer(c_int), value :: fold
+      real(c_double), value :: rhodt_next
+      type(c_ptr), value :: fluid_mask
+      type(c_ptr), value :: stream
+    end function streams_rhs_cells
     integer(c_int) function streams_reactor_batch(n_s, nbatch, w, tguess, dttry, time_end, &
         pressure, mw, rgas, cp_coeff, nreactions, kin_pack, kc_tab, num_t_tab, t_min_tab, dt_tab, &
         r_univ, tol_iter_nr, cv_coeff, nsetcv, trange, indx_cp_l, indx_cp_r, maxsteps, maxtry, tol, &

@@ -191,6 +191,7 @@ class Solver:
         epo = gridmod.ep_ord_change(nx, ny, nz, self.bctags, self.num.ep_order, self.num.weno_scheme,
                                     self.num.correct_bound_ord)
         self.t_epo = be.asarray(epo.T, "i4")
+        self._full_order = not epo.any()
         self.t_periodic = self.periodic.copy()
         # Bilger mixture fraction off (N_EoI = 1)
         self.t_eoi = be.asarray(np.ones(1))
@@ -529,10 +530,23 @@ class Solver:
                 and self.num.enable_les == 0
                 and self.be.has("rhs_sweep") and self.be.has("rhs_finish"))
 
+    def cells_supported(self) -> bool:
+        """The substep's right-hand side in one pass over the cells (streams_rhs_cells): a 3-D
+        box whose faces all take the KEEP flux of one order (no sensor, no order reduction at
+        the boundaries), nkeep = 0, sixth or eighth order throughout, NASA7 tables, and planes
+        within the kernel's 32-bit byte offsets.  Everything else takes the sweeps."""
+        n = self.num
+        ng = self.ng
+        plane = (self.nx + 2 * ng) * (self.ny + 2 * ng) * (self.nz + 2 * ng)
+        return (self._full_order and n.sensor_threshold >= 1.0 and n.nkeep == 0 and n.ep_order in (6, 8)
+                and n.visc_order == n.ep_order and min(self.nx, self.ny, self.nz) > 1 and not any(self.force_zero_flux)
+                and self.tb.indx_cp_l == 0 and plane < 1 << 29 and self.be.has("rhs_cells"))
+
     def rk_substep_fused(self, istep: int, fold_next: bool = False):
         """One RK substep in five passes: halo + aux, sensor, fused x/y/z sweeps (with
         init_flux folded into the first), and the pointwise tail (reduced viscous terms,
-        chemistry, update_flux, update_field), then the physical boundaries.  fold_next (not
+        chemistry, update_flux, update_field), then the physical boundaries; where
+        cells_supported, one pass replaces the sweeps and the tail.  fold_next (not
         for the last substep): the tail also does substep istep + 1's init_flux
         (streams_rhs_finish_next), so fl is left unset and that substep's first sweep skips
         reading it."""
@@ -551,6 +565,19 @@ class Solver:
             self.bcswap_var(jduc)
         self.bcswap_var(jdiv)
         lmax = n.ep_order // 2
+        chem = int(n.enable_chemistry == 1 and self.nr > 0)
+        if chem and getattr(self, "t_kinpack", None) is None:
+            self.t_kinpack = be.asarray(capi.kinetics_pack(tb, be.lib))
+        kin = (self.t_mw, self.t_kinpack, self.t_kc) if chem else (self.t_mw, None, None)
+        if self.cells_supported():
+            be.call("rhs_cells", self.ns, self.nx, self.ny, self.nz, self.ng, self.nv_aux, lmax, self.w, self.w_aux,
+                    self.fl, self.fln, self.cd1, self.dxi[0], self.dxi[1], self.dxi[2], self.t_x, self.t_y, self.t_z,
+                    self.t_cp, tb.nsetcv, self.t_trange, tb.indx_cp_l, tb.indx_cp_r, R_UNIV, chem, self.nr, *kin,
+                    tb.num_t_tab, tb.t_min_tab, tb.dt_tab, 2 if self._fln_set else 1, rhodt, gamdt, int(fold_next),
+                    WRAY_RHO[istep + 1] * self.dt if fold_next else 0.0, None, be.stream)
+            self._fln_set = fold_next
+            self.update_ghost()
+            return
         first = True
         for d, (nd, coord) in enumerate(zip((self.nx, self.ny, self.nz), (self.t_x, self.t_y, self.t_z))):
             if d > 0 and nd <= 1:
@@ -562,10 +589,6 @@ class Solver:
                     self.rho0, self.u0, n.flux_splitting, int(nd > 1), R_UNIV,
                     (2 if self._fln_set else 1) if first else 0, rhodt, self.fl, self.fln, be.stream)
             first = False
-        chem = int(n.enable_chemistry == 1 and self.nr > 0)
-        if chem and getattr(self, "t_kinpack", None) is None:
-            self.t_kinpack = be.asarray(capi.kinetics_pack(tb, be.lib))
-        kin = (self.t_mw, self.t_kinpack, self.t_kc) if chem else (self.t_mw, None, None)
         args = (self.ns, self.nx, self.ny, self.nz, self.ng, self.nv_aux, n.visc_order, self.w, self.w_aux, self.fl,
                 self.fln, self.cd1, self.dxi[0], self.dxi[1], self.dxi[2], 1, chem, self.nr, *kin, tb.num_t_tab,
                 tb.t_min_tab, tb.dt_tab, R_UNIV, gamdt)
