@@ -1,67 +1,110 @@
 // chem.hip — finite-rate chemistry source and the per-cell Rosenbrock integrator (FP64).
 //
-// compute_chemistry: one thread per interior cell, reaction loop over the tables in
-// their Fortran layout (arr_a(nr,2), tb_eff(nr,N_S), kc_tab(num_t_tab+1,nr), ...).
+// compute_chemistry: one thread per interior cell; the tables come in their Fortran layout
+// (arr_a(nr,2), tb_eff(nr,N_S), kc_tab(num_t_tab+1,nr), ...).
 // rosenbrock: one thread per cell restating rosenbrock_kernel with its central-difference
 // Jacobian and Crout LU; it is the FP64 yardstick for the batched integrators of reactors.hip.
 #include "chem_common.h"
+#include "kinpack.h"
+#include "thermo_dev.h"
 
 namespace streams {
 
-template <int NS>
+// The reference's dense tables are packed into one record per reaction in LDS (kinpack.h) once
+// per workgroup, each of which takes many cells: walking the dense rows costs a uniform branch
+// per species and side of every reaction (0.288 ms for 96x72x60 cells, 9 species and 21 reactions; packed 0.19 ms, bounded by the
+// exponentials and powers of the reference's rate forms, which are kept: folding b ln T into one
+// exponential with -Ea/RT takes another 0.04 ms off but has 1.2 to 1.4 times the error).
+// A mechanism with a side of more than KSIDE species, or with more records than LDS holds
+// (PACKED = false), walks the dense tables.  LO: NASA form of the tables staged in LDS, 99: any
+// other form, from global memory.
+template <int NS, int LO, bool PACKED>
 __global__ void __launch_bounds__(256) chemistry_kernel(Box b, double *__restrict__ w, double *__restrict__ w_aux,
                                                         double *__restrict__ fl, Kin K, Thermo th,
-                                                        double tol_iter_nr) {
+                                                        double tol_iter_nr, unsigned ncells) {
   using X = Idx<NS>;
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= b.fstride()) return;
-  int i = 1 + (int)(t % b.nx);
-  long r = t / b.nx;
-  int j = 1 + (int)(r % b.ny);
-  int k = 1 + (int)(r / b.ny);
-  const long pt = b.p(i, j, k), ps = b.pstride();
-  double yy[NS], conc[NS];
-  double rho = 0.0;
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    double v = w[pt + ps * s];
-    if (!(v > 0.0)) { v = 0.0; w[pt + ps * s] = 0.0; }
-    yy[s] = v;
-    rho = (s == 0) ? v : rho + v;
-  }
-  const double ri = 1.0 / rho;
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    yy[s] = yy[s] * ri;
-    w_aux[pt + ps * s] = yy[s];
-    conc[s] = rho * yy[s] / K.mw[s];
-  }
-  const double uu = w[pt + ps * (X::I_U - 1)] * ri, vv = w[pt + ps * (X::I_V - 1)] * ri;
-  const double ww = w[pt + ps * (X::I_W - 1)] * ri, rhoe = w[pt + ps * (X::I_E - 1)];
-  const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
-  const double ee = rhoe * ri - qq;
-  const double tt = temperature_from_e<NS>(ee, w_aux[pt + ps * (X::J_T - 1)], th, tol_iter_nr, yy);
-  w_aux[pt + ps * (X::J_T - 1)] = tt;
-  const double Rtti = 1.0 / (K.r_univ * tt);
-  int itt = (int)((tt - K.t_min_tab) / K.dt_tab) + 1;
-  itt = itt < 1 ? 1 : itt;
-  itt = itt > K.num_t_tab ? K.num_t_tab : itt;
-  const double ttleft = (itt - 1) * K.dt_tab + K.t_min_tab;
-  const double dtt = (tt - ttleft) / K.dt_tab;
-  double acc[NS];
-  const long fs_ = b.fstride();
-#pragma unroll
-  for (int s = 0; s < NS; ++s) acc[s] = fl[t + fs_ * s];
-  for (int lr = 0; lr < K.nr; ++lr) {
-    const double q = progress_rate<NS>(K, lr, tt, Rtti, itt, dtt, conc);
+  constexpr bool STAGED = LO != 99;
+  extern __shared__ double rec[];
+  __shared__ double tlds[STAGED ? thermo_lds_doubles<NS>(TH_CV | TH_CVH) : 1];
+  __shared__ int dense;
+  ThermoLds TL{};
+  if (threadIdx.x == 0) dense = PACKED ? 0 : 1;
+  __syncthreads();
+  if constexpr (STAGED) TL = thermo_stage<NS, LO>(th, tlds, TH_CV | TH_CVH);
+  if constexpr (PACKED)
+    for (int lr = threadIdx.x; lr < K.nr; lr += 256)
+      if (!pack_record(rec + KREC * lr, NS, lr, K.nr, K)) dense = 1;
+  __syncthreads();
+  const bool packed = dense == 0;
+  const long ps = b.pstride(), fs_ = b.fstride(), ntab = (long)K.num_t_tab + 1;
+  for (unsigned t = blockIdx.x * 256u + threadIdx.x; t < ncells; t += gridDim.x * 256u) {
+    const long pt = b.p(1 + (int)(t % b.nx), 1 + (int)(t / b.nx % b.ny), 1 + (int)(t / b.nx / b.ny));
+    double yy[NS], conc[NS], acc[NS];
+    double rho = 0.0;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      const double wdt = (K.p_co[lr + K.nr * s] - K.r_co[lr + K.nr * s]) * q * K.mw[s];
-      acc[s] = acc[s] - wdt;
+      double v = w[pt + ps * s];
+      if (!(v > 0.0)) { v = 0.0; w[pt + ps * s] = 0.0; }
+      yy[s] = v;
+      rho = (s == 0) ? v : rho + v;
     }
-  }
+    const double ri = 1.0 / rho;
 #pragma unroll
-  for (int s = 0; s < NS; ++s) fl[t + fs_ * s] = acc[s];
+    for (int s = 0; s < NS; ++s) {
+      yy[s] = yy[s] * ri;
+      w_aux[pt + ps * s] = yy[s];
+      conc[s] = rho * yy[s] / K.mw[s];
+      acc[s] = 0.0;
+    }
+    const double uu = w[pt + ps * (X::I_U - 1)] * ri, vv = w[pt + ps * (X::I_V - 1)] * ri;
+    const double ww = w[pt + ps * (X::I_W - 1)] * ri, rhoe = w[pt + ps * (X::I_E - 1)];
+    const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
+    const double ee = rhoe * ri - qq;
+    const double t0 = w_aux[pt + ps * (X::J_T - 1)];
+    double tt;
+    if constexpr (STAGED) {
+      int nrange[NS];
+      tt = temperature_from_e_lds<NS, LO>(ee, t0, TL, tol_iter_nr, yy, nrange);
+    } else {
+      tt = temperature_from_e<NS>(ee, t0, th, tol_iter_nr, yy);
+    }
+    w_aux[pt + ps * (X::J_T - 1)] = tt;
+    if (packed) {
+      const double Rtti = 1.0 / (K.r_univ * tt);
+      int itt = (int)((tt - K.t_min_tab) / K.dt_tab) + 1;
+      itt = itt < 1 ? 1 : itt;
+      itt = itt > K.num_t_tab ? K.num_t_tab : itt;
+      const double dtt = (tt - ((itt - 1) * K.dt_tab + K.t_min_tab)) / K.dt_tab;
+      for (int lr = 0; lr < K.nr; ++lr) {
+        const double *R = rec + KREC * lr;
+        auto c = [&](int s) { return conc[s]; };
+        const double q = reaction_progress<NS, true>(R, UniformInts{(const int *)R}, K.kc_tab + (itt - 1) + ntab * lr,
+                                                     tt, 0.0, Rtti, dtt, c, c);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) acc[s] = acc[s] - q * R[KD_NET + s];
+      }
+    } else {
+      chemistry_source<NS>(K, tt, conc, acc);
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) fl[t + fs_ * s] = fl[t + fs_ * s] + acc[s];
+  }
+}
+
+// workgroups of chemistry_kernel: each packs the tables once, so no more than fill the GPU
+constexpr long CHEM_BLOCKS = 1024;
+constexpr long CHEM_LDS = 64 * 1024;         // bytes of records at most
+
+template <int NS, int LO>
+void chemistry_launch(const Box &b, double *w, double *w_aux, double *fl, const Kin &K, const Thermo &th, double tol,
+                      unsigned n, hipStream_t st) {
+  long g = ((long)n + 255) / 256;
+  g = g < CHEM_BLOCKS ? g : CHEM_BLOCKS;
+  const long bytes = (long)K.nr * KREC * 8;
+  if (K.nr > 0 && bytes <= CHEM_LDS)
+    chemistry_kernel<NS, LO, true><<<(unsigned)g, 256, bytes, st>>>(b, w, w_aux, fl, K, th, tol, n);
+  else
+    chemistry_kernel<NS, LO, false><<<(unsigned)g, 256, 0, st>>>(b, w, w_aux, fl, K, th, tol, n);
 }
 
 // ------------------------------------------------------------------ Rosenbrock
@@ -113,8 +156,16 @@ extern "C" int streams_compute_chemistry(int n_s, int nx, int ny, int nz, int nv
   Kin K{mw, arr_a, arr_b, arr_ea, tb_eff, falloff_coeffs, r_coeffs, p_coeffs, kc_tab, reac_ty, isrev,
         nreactions, num_t_tab, t_min_tab, dt_tab, r_univ};
   Thermo th{cv_coeff, nullptr, trange, nsetcv, indx_cp_l, indx_cp_r};
-  STREAMS_DISPATCH_NS(n_s, (chemistry_kernel<NS><<<blocks_for(n, 256), 256, 0, as_stream(stream)>>>(
-                                b, w, w_aux, fl, K, th, tol_iter_nr)));
+  if (n > 0xfff00000l) return STREAMS_E_DIMS;  // cells are indexed with 32 bits: 290 GB of w and fl at the fewest variables
+  const bool staged = indx_cp_r == 4 && nsetcv >= 1 && nsetcv <= TMAXSET;
+  hipStream_t st = as_stream(stream);
+  if (staged && indx_cp_l == 0) {
+    STREAMS_DISPATCH_NS(n_s, (chemistry_launch<NS, 0>(b, w, w_aux, fl, K, th, tol_iter_nr, (unsigned)n, st)));
+  } else if (staged && indx_cp_l == -2) {
+    STREAMS_DISPATCH_NS(n_s, (chemistry_launch<NS, -2>(b, w, w_aux, fl, K, th, tol_iter_nr, (unsigned)n, st)));
+  } else {
+    STREAMS_DISPATCH_NS(n_s, (chemistry_launch<NS, 99>(b, w, w_aux, fl, K, th, tol_iter_nr, (unsigned)n, st)));
+  }
   return hip_status();
 }
 

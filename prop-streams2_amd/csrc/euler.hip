@@ -8,7 +8,9 @@
 //      or component-wise (Rusanov) WENO flux in fhat.  Shocked faces are a tenth of the
 //      faces in a typical shear layer but touch a third of the 64-face waves, so the
 //      list keeps the WENO lanes full instead of idling 60 % of each active wave;
-//   2. fused central pass: every face's KEEP split-form flux (or the parked WENO flux) and
+//   2. without the sensor (threshold 1 or more) and nkeep <= 0: a thread per cell and the
+//      telescoped KEEP difference (euler_cell_kernel);
+//   3. else a fused pass: every face's KEEP split-form flux (or the parked WENO flux) and
 //      the flux-difference update of fl in the same kernel, so face fluxes never round-
 //      trip through HBM:
 //        x: faces of all (j,k) lines are flattened and tiled 256 to a workgroup with a
@@ -208,6 +210,180 @@ __global__ void __launch_bounds__(128) euler_yz_fused_kernel(Box b, EulerArgs A,
   }
 }
 
+// ------------------------------------------------- cells without WENO faces
+// A direction's update of the cells whose two faces take the KEEP flux at one order: the
+// difference of the two face fluxes telescopes into the cell's own pair terms,
+// F(c) - F(c-1) = sum_l c_l [G(c, c+l) - G(c-l, c)] (cells.hip), so one thread per cell needs no
+// neighbour's flux, and every cell is a thread of its own: the column march runs nx*nz*ny/16
+// threads, too few to hide its loads (96x72x60 cells, 9 species, sixth order: x 0.092 -> 0.059 ms, y
+// 0.40 -> 0.062, z 0.40 -> 0.077).  Bounded by the loads of the L1: 16 clocks of a CU per wave's
+// load, seven cells of each variable.  Any order takes this form: the loads of the levels above
+// lmax are skipped.  Cells beside an order-reduced or zeroed face
+// are left to euler_edge_kernel.  nkeep <= 0.
+template <int DIR>
+__device__ inline bool cell_of_sweep(const Box &b, const EulerArgs &A, unsigned t, int &t1, int &t2, int &c) {
+  // x: the cell fastest; y, z: i fastest, then the other index, then the cell
+  const unsigned nc = (unsigned)(A.fe - A.fs), n1 = DIR == 1 ? nc : (unsigned)b.nx;
+  const unsigned n2 = DIR == 1 ? (unsigned)b.ny : DIR == 2 ? nc : (unsigned)b.ny;
+  const unsigned x = t % n1, r = t / n1, y = r % n2, z = r / n2;
+  if (DIR == 1) { c = A.fs + 1 + (int)x; t1 = 1 + (int)y; t2 = 1 + (int)z; }
+  else if (DIR == 2) { t1 = 1 + (int)x; c = A.fs + 1 + (int)y; t2 = 1 + (int)z; }
+  else { t1 = 1 + (int)x; t2 = 1 + (int)y; c = A.fs + 1 + (int)z; }
+  return z < (DIR == 3 ? nc : (unsigned)b.nz);
+}
+template <int DIR>
+__device__ inline long sweep_cell_index(const Box &b, int t1, int t2, int c) {
+  return DIR == 1 ? b.f(c, t1, t2) : DIR == 2 ? b.f(t1, c, t2) : b.f(t1, t2, c);
+}
+// order of both faces when they share it and neither is zeroed, else 0
+template <int DIR>
+__device__ inline int cell_order(const Box &b, const EulerArgs &A, int t1, int t2, int c) {
+  const int el = epo_at<DIR>(b, A.epo, t1, t2, c - 1), er = epo_at<DIR>(b, A.epo, t1, t2, c);
+  int lmax = A.lmax_base + el;
+  lmax = lmax < 1 ? 1 : lmax;
+  const bool zero = (c == 1 && A.zmin == 1) || (c == A.n && A.zmax == 1);
+  return el == er && !zero ? lmax : 0;
+}
+
+template <int NS, int DIR>
+__global__ void __launch_bounds__(256) euler_cell_kernel(Box b, EulerArgs A) {
+  using X = Idx<NS>;
+  constexpr int LB = 4;
+  int t1, t2, c;
+  if (!cell_of_sweep<DIR>(b, A, blockIdx.x * 256u + threadIdx.x, t1, t2, c)) return;
+  const int lmax = cell_order<DIR>(b, A, t1, t2, c);
+  if (lmax == 0) return;
+  Line L{A.w_aux, 0, 0, b.pstride()};
+  line_base<DIR>(b, t1, t2, L.base, L.st);
+  const double met = A.metric[c - 1];
+  const long fc = sweep_cell_index<DIR>(b, t1, t2, c), fs_ = b.fstride();
+  double P[2 * LB], psum = 0.0;
+  {
+    const double rc = L(c, X::J_R), pc = L(c, X::J_P), hc = L(c, X::J_H);
+    const double vc[3] = {L(c, X::J_U), L(c, X::J_V), L(c, X::J_W)};
+    const bool split = A.nkeep >= 0;
+    const double ec = split ? hc - pc / rc - 0.5 * (vc[0] * vc[0] + vc[1] * vc[1] + vc[2] * vc[2]) : hc;
+    double m[3] = {0.0, 0.0, 0.0}, e = 0.0;
+#pragma unroll
+    for (int l = 1; l <= LB; ++l) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        double f = 0.0;
+        if (l <= lmax) {
+          const int q = s == 0 ? c + l : c - l;
+          const double cl = (s == 0 ? met : -met) * A.cd1[(l - 1) + 4 * (lmax - 1)];
+          const double rn = L(q, X::J_R), pn = L(q, X::J_P), hn = L(q, X::J_H);
+          const double vn[3] = {L(q, X::J_U), L(q, X::J_V), L(q, X::J_W)};
+          f = 0.25 * cl * (rc + rn) * (vc[DIR - 1] + vn[DIR - 1]);
+          m[0] += f * (vc[0] + vn[0]);
+          m[1] += f * (vc[1] + vn[1]);
+          m[2] += f * (vc[2] + vn[2]);
+          m[DIR - 1] += cl * (pc + pn);
+          if (split) {
+            const double en = hn - pn / rn - 0.5 * (vn[0] * vn[0] + vn[1] * vn[1] + vn[2] * vn[2]);
+            e += f * (ec + en + (vc[0] * vn[0] + vc[1] * vn[1] + vc[2] * vn[2]));
+            e += cl * (vc[DIR - 1] * pn + vn[DIR - 1] * pc);
+          } else {
+            e += f * (hc + hn);
+          }
+        }
+        P[2 * (l - 1) + s] = f;
+        psum += f;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) A.fl[fc + fs_ * (NS + q)] += m[q];
+    A.fl[fc + fs_ * (NS + 3)] += e;
+  }
+#pragma unroll 3
+  for (int s = 0; s < NS; ++s) {
+    double acc = psum * L(c, s + 1);
+#pragma unroll
+    for (int l = 1; l <= LB; ++l)
+      if (l <= lmax) acc += P[2 * (l - 1)] * L(c + l, s + 1) + P[2 * l - 1] * L(c - l, s + 1);
+    A.fl[fc + fs_ * s] += acc;
+  }
+}
+
+// The cells euler_cell_kernel leaves: both face fluxes in full, each at its own order; a
+// zeroed face keeps its pressure alone.  Every pair of the highest order is an unrolled, predicated term, so lanes of
+// different order share one instruction stream.
+template <int NS, int DIR>
+__global__ void __launch_bounds__(256) euler_edge_kernel(Box b, EulerArgs A) {
+  using X = Idx<NS>;
+  constexpr int LB = 4, NP = LB * (LB + 1) / 2;
+  int t1, t2, c;
+  if (!cell_of_sweep<DIR>(b, A, blockIdx.x * 256u + threadIdx.x, t1, t2, c)) return;
+  if (cell_order<DIR>(b, A, t1, t2, c) != 0) return;
+  Line L{A.w_aux, 0, 0, b.pstride()};
+  line_base<DIR>(b, t1, t2, L.base, L.st);
+  const double met = A.metric[c - 1];
+  const long fc = sweep_cell_index<DIR>(b, t1, t2, c), fs_ = b.fstride();
+  double P[2][NP], m[2][3], e[2];
+  int lo = 0, hi = 0;                        // cells c - lo .. c + hi take part
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int f = c - 1 + s;
+    int lmax = A.lmax_base + epo_at<DIR>(b, A.epo, t1, t2, f);
+    lmax = lmax < 1 ? 1 : lmax;
+    const bool zero = (f == 0 && A.zmin == 1) || (f == A.n && A.zmax == 1);
+    const int lf = zero ? 0 : lmax;
+    lo = lo > lf - s ? lo : lf - s;
+    hi = hi > lf - 1 + s ? hi : lf - 1 + s;
+    m[s][0] = m[s][1] = m[s][2] = e[s] = 0.0;
+#pragma unroll
+    for (int l = 1; l <= LB; ++l) {
+#pragma unroll
+      for (int q = 0; q < l; ++q) {
+        double pf = 0.0;
+        if (l <= lmax) {
+          const int a = f - q, z = f - q + l;
+          const double cl = A.cd1[(l - 1) + 4 * (lmax - 1)];
+          const double ra = L(a, X::J_R), pa = L(a, X::J_P), ha = L(a, X::J_H);
+          const double rz = L(z, X::J_R), pz = L(z, X::J_P), hz = L(z, X::J_H);
+          const double va[3] = {L(a, X::J_U), L(a, X::J_V), L(a, X::J_W)};
+          const double vz[3] = {L(z, X::J_U), L(z, X::J_V), L(z, X::J_W)};
+          m[s][DIR - 1] += cl * (pa + pz);
+          if (!zero) {
+            pf = 0.25 * cl * (ra + rz) * (va[DIR - 1] + vz[DIR - 1]);
+            for (int d = 0; d < 3; ++d) m[s][d] += pf * (va[d] + vz[d]);
+            if (A.nkeep >= 0) {
+              const double ea = ha - pa / ra - 0.5 * (va[0] * va[0] + va[1] * va[1] + va[2] * va[2]);
+              const double ez = hz - pz / rz - 0.5 * (vz[0] * vz[0] + vz[1] * vz[1] + vz[2] * vz[2]);
+              e[s] += pf * (ea + ez + (va[0] * vz[0] + va[1] * vz[1] + va[2] * vz[2]));
+              e[s] += cl * (va[DIR - 1] * pz + vz[DIR - 1] * pa);
+            } else {
+              e[s] += pf * (ha + hz);
+            }
+          }
+        }
+        P[s][l * (l - 1) / 2 + q] = pf;
+      }
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < 3; ++d) A.fl[fc + fs_ * (NS + d)] += (m[1][d] - m[0][d]) * met;
+  A.fl[fc + fs_ * (NS + 3)] += (e[1] - e[0]) * met;
+#pragma unroll 1
+  for (int s = 0; s < NS; ++s) {
+    double y[2 * LB + 1], F[2] = {0.0, 0.0};
+#pragma unroll
+    for (int q = -LB; q <= LB; ++q) y[q + LB] = q >= -lo && q <= hi ? L(c + q, s + 1) : 0.0;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+      for (int l = 1; l <= LB; ++l) {
+#pragma unroll
+        for (int q = 0; q < l; ++q) {
+          const int a = k - 1 - q;             // cells c + a and c + a + l
+          F[k] += P[k][l * (l - 1) / 2 + q] * (y[a + LB] + y[a + l + LB]);
+        }
+      }
+    }
+    A.fl[fc + fs_ * s] += (F[1] - F[0]) * met;
+  }
+}
+
 template <int NS, int DIR>
 inline int prepass_launch(const Box &b, const EulerArgs &A, int t1n, long nfaces, hipStream_t st) {
   if (nfaces > (long)0xFFFFFF00u) return STREAMS_E_DIMS;
@@ -252,6 +428,11 @@ int euler_launch(const Box &b, EulerArgs A, hipStream_t st) {
   if (check) {
     int rc = prepass_launch<NS, DIR>(b, A, t1n, nfaces, st);
     if (rc) return rc;
+  } else if (A.nkeep <= 0 && (long)(nf - 1) * t1n * t2n < 0xffffff00l) {
+    const unsigned g = blocks_for((long)(nf - 1) * t1n * t2n, 256);
+    euler_cell_kernel<NS, DIR><<<g, 256, 0, st>>>(b, A);
+    euler_edge_kernel<NS, DIR><<<g, 256, 0, st>>>(b, A);
+    return hip_status();
   }
   if (DIR == 1) {
     long nblk = (nfaces - 1 + (XT - 2)) / (XT - 1);

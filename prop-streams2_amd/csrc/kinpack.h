@@ -68,18 +68,6 @@ __device__ inline void record_coeffs(kdouble *R, kint *I, int nre, int npr, doub
 
 template <int S, int NS>
 struct RefSpecies {
-  // q1 = prod c^r, q2 = prod c^p in ascending species order with the reference's
-  // exponent cases (1: multiply, other non-zero: pow)
-  __device__ static inline void products(kdouble *R, kint *I, int nre, int npr, const double *conc, double &q1,
-                                         double &q2) {
-    double rr, pp;
-    record_coeffs<S>(R, I, nre, npr, rr, pp);
-    if (rr == 1.0) q1 = q1 * conc[S];
-    else if (rr != 0.0) q1 = q1 * pow(conc[S], rr);
-    if (pp == 1.0) q2 = q2 * conc[S];
-    else if (pp != 0.0) q2 = q2 * pow(conc[S], pp);
-    RefSpecies<S + 1, NS>::products(R, I, nre, npr, conc, q1, q2);
-  }
   // acc_s -= ((p - r) q) W_s for the species of the reaction
   __device__ static inline void accumulate(kdouble *R, kint *I, int nre, int npr, double q, const double *mw,
                                            double *acc) {
@@ -91,35 +79,46 @@ struct RefSpecies {
 };
 template <int NS>
 struct RefSpecies<NS, NS> {
-  __device__ static inline void products(kdouble *, kint *, int, int, const double *, double &, double &) {}
   __device__ static inline void accumulate(kdouble *, kint *, int, int, double, const double *, double *) {}
 };
 
-// Rate of progress of one reaction in the forms of REF = false.  The record and conc(s) are
+// Rate of progress of one reaction (REF: see chemistry_source_from).  The record and conc(s) are
 // read through the caller's pointers: wave-uniform scalar loads when every lane walks the same
 // reaction, vector loads when each lane takes its own.  kc points at K_c's table row.  pick(s)
-// is conc(s) where s comes from the record (a register array would be indexed dynamically).
-template <int NS, class RD, class RI, class Conc, class Pick>
+// is conc(s) where s comes from the record (a register array would be indexed dynamically); a
+// side's species are in ascending order.
+template <int NS, bool REF = false, class RD, class RI, class Conc, class Pick>
 __device__ inline double reaction_progress(RD R, RI I, const double *kc, double tt, double lnT, double Rtti, double dtt,
                                            const Conc &conc, const Pick &pick) {
   constexpr double LN10 = 2.302585092994045684;
   constexpr double ILN10 = 0.434294481903251827651;
+  auto arrhenius = [&](int k) {
+    if constexpr (REF) return R[k] * pow(tt, R[k + 1]) * exp(-R[k + 2] * Rtti);
+    else return R[k] * exp(R[k + 1] * lnT - R[k + 2] * Rtti);
+  };
+  auto lg = [&](double x) {
+    if constexpr (REF) return log10(x);
+    else return log(x) * ILN10;
+  };
+  auto third_body = [&] {
+    double tb = 0.0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) tb = tb + R[KD_TB + s] * conc(s);
+    return tb;
+  };
   const int ty = I[KI_TY];
   double kf, tbv = 1.0;
   if (ty <= 1) {
     kf = R[KD_A];
-    if (I[KI_ARR]) kf = kf * exp(R[KD_A + 1] * lnT - R[KD_A + 2] * Rtti);
-    if (ty == 1) {
-      tbv = 0.0;
-#pragma unroll
-      for (int s = 0; s < NS; ++s) tbv = tbv + R[KD_TB + s] * conc(s);
+    if constexpr (REF) {
+      if (R[KD_A + 1] != 0.0) kf = kf * pow(tt, R[KD_A + 1]);
+      if (R[KD_A + 2] != 0.0) kf = kf * exp(-R[KD_A + 2] * Rtti);
+    } else {
+      if (I[KI_ARR]) kf = kf * exp(R[KD_A + 1] * lnT - R[KD_A + 2] * Rtti);
     }
+    if (ty == 1) tbv = third_body();
   } else {
-    const double k0 = R[KD_A] * exp(R[KD_A + 1] * lnT - R[KD_A + 2] * Rtti);
-    const double kinf = R[KD_AINF] * exp(R[KD_AINF + 1] * lnT - R[KD_AINF + 2] * Rtti);
-    double tb = 0.0;
-#pragma unroll
-    for (int s = 0; s < NS; ++s) tb = tb + R[KD_TB + s] * conc(s);
+    const double k0 = arrhenius(KD_A), kinf = arrhenius(KD_AINF), tb = third_body();
     const double rpres = k0 * tb / kinf;
     if (ty == 2) {
       kf = kinf * (rpres / (1.0 + rpres));
@@ -129,18 +128,22 @@ __device__ inline double reaction_progress(RD R, RI I, const double *kc, double 
       } else {
         double fcent = (1.0 - R[KD_FC]) * exp(-tt / R[KD_FC + 1]) + R[KD_FC] * exp(-tt / R[KD_FC + 2]);
         if (I[KI_T2]) fcent = fcent + exp(-R[KD_FC + 3] / tt);
-        fcent = log(fcent) * ILN10;
+        fcent = lg(fcent);
         const double coff = -0.4 - 0.67 * fcent;
         const double noff = 0.75 - 1.27 * fcent;
-        const double lr10 = log(rpres) * ILN10;
+        const double lr10 = lg(rpres);
         const double fo = (lr10 + coff) / (noff - 0.14 * (lr10 + coff));
-        kf = kinf * (rpres / (1.0 + rpres)) * exp(LN10 * (fcent / (1.0 + fo * fo)));
+        double foff;
+        if constexpr (REF) foff = pow(10.0, pow(1.0 + pow(fo, 2.0), -1.0) * fcent);
+        else foff = exp(LN10 * (fcent / (1.0 + fo * fo)));
+        kf = kinf * (rpres / (1.0 + rpres)) * foff;
       }
     } else {
-      const double l10 = log(rpres) * ILN10;
-      const double xoff = 1.0 / (1.0 + l10 * l10);
+      const double l10 = lg(rpres);
       const double sri = R[KD_FC] * exp(-R[KD_FC + 1] / tt) + exp(-tt / R[KD_FC + 2]);
-      const double foff = R[KD_FC + 3] * exp(xoff * log(sri)) * exp(R[KD_FC + 4] * lnT);
+      double foff;
+      if constexpr (REF) foff = R[KD_FC + 3] * pow(sri, 1.0 / (1.0 + pow(l10, 2.0))) * pow(tt, R[KD_FC + 4]);
+      else foff = R[KD_FC + 3] * exp(1.0 / (1.0 + l10 * l10) * log(sri)) * exp(R[KD_FC + 4] * lnT);
       kf = kinf * (rpres / (1.0 + rpres)) * foff;
     }
   }
@@ -149,14 +152,18 @@ __device__ inline double reaction_progress(RD R, RI I, const double *kc, double 
     const DoublePair k = load_pair(kc);
     kb = kf / (k.a + (k.b - k.a) * dtt);
   }
+  auto power = [&](double c, double ex) {
+    if constexpr (REF) return ex == 1.0 ? c : pow(c, ex);
+    else return conc_power(c, ex);
+  };
   double q1 = 1.0, q2 = 1.0;
   const int nre = I[KI_NRE], npr = I[KI_NPR];
 #pragma unroll
   for (int e = 0; e < KSIDE; ++e)
-    if (e < nre) q1 = q1 * conc_power(pick(I[KI_RE + e]), R[KD_REX + e]);
+    if (e < nre) q1 = q1 * power(pick(I[KI_RE + e]), R[KD_REX + e]);
 #pragma unroll
   for (int e = 0; e < KSIDE; ++e)
-    if (e < npr) q2 = q2 * conc_power(pick(I[KI_PR + e]), R[KD_PEX + e]);
+    if (e < npr) q2 = q2 * power(pick(I[KI_PR + e]), R[KD_PEX + e]);
   return tbv * (kf * q1 - kb * q2);
 }
 
@@ -189,55 +196,8 @@ __device__ inline void chemistry_source_from(const KinPacked &K, double tt, cons
     kint *I = (kint *)R;
     const double *kp = K.kc_tab + (itt - 1) + ntab * lr;
     if (REF) {
-      const int ty = I[KI_TY];
-      double kf, tbv = 1.0;
-      if (ty <= 1) {
-        kf = R[KD_A];
-        if (R[KD_A + 1] != 0.0) kf = kf * pow(tt, R[KD_A + 1]);
-        if (R[KD_A + 2] != 0.0) kf = kf * exp(-R[KD_A + 2] * Rtti);
-        if (ty == 1) {
-          tbv = 0.0;
-#pragma unroll
-          for (int s = 0; s < NS; ++s) tbv = tbv + R[KD_TB + s] * conc[s];
-        }
-      } else {
-        const double k0 = R[KD_A] * pow(tt, R[KD_A + 1]) * exp(-R[KD_A + 2] * Rtti);
-        const double kinf = R[KD_AINF] * pow(tt, R[KD_AINF + 1]) * exp(-R[KD_AINF + 2] * Rtti);
-        double tb = 0.0;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) tb = tb + R[KD_TB + s] * conc[s];
-        const double rpres = k0 * tb / kinf;
-        if (ty == 2) {
-          kf = kinf * (rpres / (1.0 + rpres));
-        } else if (ty == 3) {
-          if (rpres < 1e-30) {
-            kf = k0 * tb;
-          } else {
-            double fcent = (1.0 - R[KD_FC]) * exp(-tt / R[KD_FC + 1]) + R[KD_FC] * exp(-tt / R[KD_FC + 2]);
-            if (I[KI_T2]) fcent = fcent + exp(-R[KD_FC + 3] / tt);
-            fcent = log10(fcent);
-            const double coff = -0.4 - 0.67 * fcent;
-            const double noff = 0.75 - 1.27 * fcent;
-            const double doff = 0.14;
-            const double lr10 = log10(rpres);
-            const double fo = (lr10 + coff) / (noff - doff * (lr10 + coff));
-            const double foff = pow(10.0, pow(1.0 + pow(fo, 2.0), -1.0) * fcent);
-            kf = kinf * (rpres / (1.0 + rpres)) * foff;
-          }
-        } else {
-          const double xoff = 1.0 / (1.0 + pow(log10(rpres), 2.0));
-          const double foff = R[KD_FC + 3] * pow(R[KD_FC] * exp(-R[KD_FC + 1] / tt) + exp(-tt / R[KD_FC + 2]), xoff) *
-                              pow(tt, R[KD_FC + 4]);
-          kf = kinf * (rpres / (1.0 + rpres)) * foff;
-        }
-      }
-      double kb = 0.0;
-      if (I[KI_REV] == 1) kb = kf / (kp[0] + (kp[1] - kp[0]) * dtt);
-      double q1 = 1.0, q2 = 1.0;
-      const int nre = I[KI_NRE], npr = I[KI_NPR];
-      RefSpecies<0, NS>::products(R, I, nre, npr, conc, q1, q2);
-      const double q = tbv * (kf * q1 - kb * q2);
-      RefSpecies<0, NS>::accumulate(R, I, nre, npr, q, mw, acc);
+      const double q = reaction_progress<NS, true>(R, I, kp, tt, 0.0, Rtti, dtt, [&](int s) { return conc[s]; }, pick);
+      RefSpecies<0, NS>::accumulate(R, I, I[KI_NRE], I[KI_NPR], q, mw, acc);
     } else {
       const double q = reaction_progress<NS>(R, I, kp, tt, lnT, Rtti, dtt, [&](int s) { return conc[s]; }, pick);
 #pragma unroll
@@ -251,5 +211,48 @@ __device__ inline void chemistry_source_packed(const KinPacked &K, double tt, co
                                                const double *mw = nullptr) {
   chemistry_source_from<NS, REF>(K, tt, conc, acc, mw, [&](int s) { return conc[s]; });
 }
+
+// One reaction's record from the dense tables (the layout above); false when a side has more
+// than KSIDE species.
+template <class Dense>
+__device__ inline bool pack_record(double *R, int n_s, int lr, int nr, const Dense &K) {
+  for (int q = 0; q < KREC; ++q) R[q] = 0.0;
+  int *I = reinterpret_cast<int *>(R);
+  I[KI_TY] = K.reac_ty[lr];
+  I[KI_REV] = K.isrev[lr];
+  int nre = 0, npr = 0;
+  bool fits = true;
+  for (int s = 0; s < n_s; ++s) {
+    const double rr = K.r_co[lr + nr * s], pp = K.p_co[lr + nr * s];
+    if (rr != 0.0) {
+      if (nre == KSIDE) fits = false;
+      else { I[KI_RE + nre] = s; R[KD_REX + nre] = rr; ++nre; }
+    }
+    if (pp != 0.0) {
+      if (npr == KSIDE) fits = false;
+      else { I[KI_PR + npr] = s; R[KD_PEX + npr] = pp; ++npr; }
+    }
+    R[KD_NET + s] = (pp - rr) * K.mw[s];
+    R[KD_TB + s] = K.tb_eff[lr + nr * s];
+  }
+  I[KI_NRE] = nre;
+  I[KI_NPR] = npr;
+  I[KI_ARR] = (K.arr_b[lr] != 0.0 || K.arr_ea[lr] != 0.0) ? 1 : 0;
+  R[KD_A] = K.arr_a[lr];
+  R[KD_A + 1] = K.arr_b[lr];
+  R[KD_A + 2] = K.arr_ea[lr];
+  R[KD_AINF] = K.arr_a[lr + nr];
+  R[KD_AINF + 1] = K.arr_b[lr + nr];
+  R[KD_AINF + 2] = K.arr_ea[lr + nr];
+  for (int q = 0; q < 5; ++q) R[KD_FC + q] = K.falloff[lr + nr * q];
+  I[KI_T2] = K.falloff[lr + 3 * nr] != -3.14 ? 1 : 0;
+  return fits;
+}
+
+// The same for all lanes, as a scalar.
+struct UniformInts {
+  const int *p;
+  __device__ inline int operator[](int i) const { return __builtin_amdgcn_readfirstlane(p[i]); }
+};
 
 }  // namespace streams
