@@ -37,6 +37,9 @@ FILE_FLAGS = {
     "finish.hip": ["-mllvm", "-disable-machine-licm"],
     "reactors_group.hip": ["-mllvm", "-disable-machine-licm"],
     "reactors_group_cp.hip": ["-mllvm", "-disable-machine-licm"],
+    "reactors_ref.hip": ["-mllvm", "-disable-machine-licm"],
+    "reactors_ref_cp.hip": ["-mllvm", "-disable-machine-licm"],
+    "rosenbrock.hip": ["-mllvm", "-disable-machine-licm"],
     "euler.hip": ["-ffp-contract=off"],
 }
 

@@ -2,8 +2,8 @@
 //
 // compute_chemistry: one thread per interior cell; the tables come in their Fortran layout
 // (arr_a(nr,2), tb_eff(nr,N_S), kc_tab(num_t_tab+1,nr), ...).
-// rosenbrock: one thread per cell restating rosenbrock_kernel with its central-difference
-// Jacobian and Crout LU; it is the FP64 yardstick for the batched integrators of reactors.hip.
+// rosenbrock: rosenbrock_kernel with its central-difference Jacobian and Crout LU, a row of lanes
+// per cell (rosenbrock.hip) or, for tables that do not fit its records, one thread per cell.
 #include "chem_common.h"
 #include "kinpack.h"
 #include "thermo_dev.h"
@@ -12,9 +12,10 @@ namespace streams {
 
 // The reference's dense tables are packed into one record per reaction in LDS (kinpack.h) once
 // per workgroup, each of which takes many cells: walking the dense rows costs a uniform branch
-// per species and side of every reaction (0.288 ms for 96x72x60 cells, 9 species and 21 reactions; packed 0.19 ms, bounded by the
-// exponentials and powers of the reference's rate forms, which are kept: folding b ln T into one
-// exponential with -Ea/RT takes another 0.04 ms off but has 1.2 to 1.4 times the error).
+// per species and side of every reaction (0.288 ms for 96x72x60 cells, 9 species and
+// 21 reactions; packed 0.19 ms, bounded by the exponentials and powers of the reference's rate
+// forms, which are kept: folding b ln T into one exponential with -Ea/RT takes another 0.04 ms off
+// but has 1.2 to 1.4 times the error).
 // A mechanism with a side of more than KSIDE species, or with more records than LDS holds
 // (PACKED = false), walks the dense tables.  LO: NASA form of the tables staged in LDS, 99: any
 // other form, from global memory.
@@ -108,16 +109,31 @@ void chemistry_launch(const Box &b, double *w, double *w_aux, double *fl, const 
 }
 
 // ------------------------------------------------------------------ Rosenbrock
+int rosenbrock_rows(int n_s, const Box &b, double *w, double *w_aux, const Kin &K, const Thermo &th,
+                    double tol_iter_nr, double dttry, double time_start, double time_end, int maxsteps, int maxtry,
+                    double tol, const Pasr &pasr, hipStream_t st);
+// Cells above which one lane per cell fills the GPU (256 CUs x 2 waves per SIMD), and the idle
+// lanes of a row's Newton chain cost more than the scratch of a lane's Jacobian: random states, one
+// interval of 2 ns, 28800 cells of 9 species 67.7 -> 33.0 ms, 115200 cells of 14 species 450 ->
+// 378, but 414720 cells of 9 species 320 -> 398.
+constexpr long ROWS_CELLS = 131072;
+constexpr long ROWS_LDS = 36 * 1024;         // bytes of records at most, beside the rows' own 24 KB
+
 // 2 waves per SIMD (the compiler's own choice is 1, with 2.8-3.7 KB of per-lane spills):
 // the extra resident wave hides the spill latency (one integration of a 128^3 box at 1500 K,
-// 87.3 -> 67.2 ms; 3 waves: 92.9 ms; bit-identical)
+// 87.3 -> 67.2 ms; 3 waves: 92.9 ms; bit-identical).  rows: rosenbrock_rows was launched and
+// takes the call if every side of the reactions fits its records.
 template <int NS>
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) rosenbrock_kernel(Box b, double *__restrict__ w, double *__restrict__ w_aux,
-                                                         Kin K, Thermo th, double tol_iter_nr, double dttry,
-                                                         double time_start, double time_end, int maxsteps,
-                                                         int maxtry, double tol, Pasr pasr) {
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
+rosenbrock_kernel(Box b, double *__restrict__ w, double *__restrict__ w_aux, Kin K, Thermo th, double tol_iter_nr,
+                  double dttry, double time_start, double time_end, int maxsteps, int maxtry, double tol, Pasr pasr,
+                  bool rows) {
   using X = Idx<NS>;
   constexpr int NV = NS + 4;
+  if (rows) {
+    __shared__ int flag;
+    if (sides_fit(NS, K, &flag)) return;
+  }
   long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= b.fstride()) return;
   int i = 1 + (int)(t % b.nx);
@@ -156,7 +172,8 @@ extern "C" int streams_compute_chemistry(int n_s, int nx, int ny, int nz, int nv
   Kin K{mw, arr_a, arr_b, arr_ea, tb_eff, falloff_coeffs, r_coeffs, p_coeffs, kc_tab, reac_ty, isrev,
         nreactions, num_t_tab, t_min_tab, dt_tab, r_univ};
   Thermo th{cv_coeff, nullptr, trange, nsetcv, indx_cp_l, indx_cp_r};
-  if (n > 0xfff00000l) return STREAMS_E_DIMS;  // cells are indexed with 32 bits: 290 GB of w and fl at the fewest variables
+  // cells are indexed with 32 bits: w, w_aux and fl of more would not fit the memory
+  if (n > 0xfff00000l) return STREAMS_E_DIMS;
   const bool staged = indx_cp_r == 4 && nsetcv >= 1 && nsetcv <= TMAXSET;
   hipStream_t st = as_stream(stream);
   if (staged && indx_cp_l == 0) {
@@ -191,8 +208,16 @@ extern "C" int streams_rosenbrock(int n_s, int nv, int nv_aux, int nx, int ny, i
   Kin K{mw, arr_a, arr_b, arr_ea, tb_eff, falloff_coeffs, r_coeffs, p_coeffs, kc_tab, reac_ty, isrev,
         nreactions, num_t_tab, t_min_tab, dt_tab, r_univ};
   Thermo th{cv_coeff, nullptr, trange, nsetcv, indx_cp_l, indx_cp_r};
-  STREAMS_DISPATCH_NS(n_s, (rosenbrock_kernel<NS><<<blocks_for(n, 128), 128, 0, as_stream(stream)>>>(
+  const bool rows = (indx_cp_l == 0 || indx_cp_l == -2) && indx_cp_r == 4 && (long)nreactions * KREC * 8 <= ROWS_LDS &&
+                    n <= ROWS_CELLS;
+  hipStream_t st = as_stream(stream);
+  if (rows) {
+    const int rc = rosenbrock_rows(n_s, b, w, w_aux, K, th, tol_iter_nr, dttry, time_start, time_end, maxsteps,
+                                   maxtry, tol, pasr, st);
+    if (rc) return rc;
+  }
+  STREAMS_DISPATCH_NS(n_s, (rosenbrock_kernel<NS><<<blocks_for(n, 128), 128, 0, st>>>(
                                 b, w, w_aux, K, th, tol_iter_nr, dttry, time_start, time_end, maxsteps, maxtry,
-                                tol, pasr)));
+                                tol, pasr, rows)));
   return hip_status();
 }

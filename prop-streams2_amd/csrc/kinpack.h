@@ -55,8 +55,8 @@ __device__ inline double conc_power(double c, double ex) {
 
 // The record's (reactant, product) exponents of species s (0 when s does not take part):
 // the values of r_coeffs(lr,s) and p_coeffs(lr,s).
-template <int S>
-__device__ inline void record_coeffs(kdouble *R, kint *I, int nre, int npr, double &rr, double &pp) {
+template <int S, class RD, class RI>
+__device__ inline void record_coeffs(RD R, RI I, int nre, int npr, double &rr, double &pp) {
   rr = 0.0;
   pp = 0.0;
 #pragma unroll
@@ -69,8 +69,8 @@ __device__ inline void record_coeffs(kdouble *R, kint *I, int nre, int npr, doub
 template <int S, int NS>
 struct RefSpecies {
   // acc_s -= ((p - r) q) W_s for the species of the reaction
-  __device__ static inline void accumulate(kdouble *R, kint *I, int nre, int npr, double q, const double *mw,
-                                           double *acc) {
+  template <class RD, class RI>
+  __device__ static inline void accumulate(RD R, RI I, int nre, int npr, double q, const double *mw, double *acc) {
     double rr, pp;
     record_coeffs<S>(R, I, nre, npr, rr, pp);
     if (rr != 0.0 || pp != 0.0) acc[S] = acc[S] - ((pp - rr) * q) * mw[S];
@@ -79,7 +79,8 @@ struct RefSpecies {
 };
 template <int NS>
 struct RefSpecies<NS, NS> {
-  __device__ static inline void accumulate(kdouble *, kint *, int, int, double, const double *, double *) {}
+  template <class RD, class RI>
+  __device__ static inline void accumulate(RD, RI, int, int, double, const double *, double *) {}
 };
 
 // Rate of progress of one reaction (REF: see chemistry_source_from).  The record and conc(s) are
@@ -167,6 +168,12 @@ __device__ inline double reaction_progress(RD R, RI I, const double *kc, double 
   return tbv * (kf * q1 - kb * q2);
 }
 
+// The same for all lanes, as a scalar.
+struct UniformInts {
+  const int *p;
+  __device__ inline int operator[](int i) const { return __builtin_amdgcn_readfirstlane(p[i]); }
+};
+
 // Species source -omega_s W_s accumulated into acc[0..NS) for one cell at temperature tt
 // with molar concentrations conc (compute_chemistry_cuf's reaction loop,
 // kernels_gpu.F90:9551-9649).
@@ -179,9 +186,10 @@ __device__ inline double reaction_progress(RD R, RI I, const double *kc, double 
 //    with the b = 0 and Ea = 0 cases skipped, log10, pow(10, .), pow for exponents other
 //    than 1, products over the species in ascending order, acc -= ((p - r) q) W_s with
 //    mw = W_s.
-template <int NS, bool REF, class Pick>
+//  * LDSREC: the records are read from LDS (pack) instead of K.pack.
+template <int NS, bool REF, bool LDSREC = false, class Pick>
 __device__ inline void chemistry_source_from(const KinPacked &K, double tt, const double *conc, double *acc,
-                                             const double *mw, const Pick &pick) {
+                                             const double *mw, const Pick &pick, const double *pack = nullptr) {
   static_assert(NS <= KTB, "third-body efficiencies of a record hold at most KTB species");
   const double Rtti = 1.0 / (K.r_univ * tt);
   const double lnT = log(tt);
@@ -192,8 +200,16 @@ __device__ inline void chemistry_source_from(const KinPacked &K, double tt, cons
   const double dtt = (tt - ttleft) / K.dt_tab;
   const long ntab = (long)K.num_t_tab + 1;
   for (int lr = 0; lr < K.nr; ++lr) {
-    kdouble *R = (kdouble *)K.pack + KREC * lr;
-    kint *I = (kint *)R;
+    auto record = [&] {
+      if constexpr (LDSREC) return pack + KREC * lr;
+      else return (kdouble *)K.pack + KREC * lr;
+    };
+    auto R = record();
+    auto ints = [&] {
+      if constexpr (LDSREC) return UniformInts{(const int *)R};
+      else return (kint *)R;
+    };
+    auto I = ints();
     const double *kp = K.kc_tab + (itt - 1) + ntab * lr;
     if (REF) {
       const double q = reaction_progress<NS, true>(R, I, kp, tt, 0.0, Rtti, dtt, [&](int s) { return conc[s]; }, pick);
@@ -249,10 +265,21 @@ __device__ inline bool pack_record(double *R, int n_s, int lr, int nr, const Den
   return fits;
 }
 
-// The same for all lanes, as a scalar.
-struct UniformInts {
-  const int *p;
-  __device__ inline int operator[](int i) const { return __builtin_amdgcn_readfirstlane(p[i]); }
-};
+// false when a side of a reaction has more than KSIDE species (all threads of the block call)
+template <class Dense>
+__device__ inline bool sides_fit(int n_s, const Dense &K, int *flag) {
+  if (threadIdx.x == 0) *flag = 1;
+  __syncthreads();
+  for (int lr = threadIdx.x; lr < K.nr; lr += blockDim.x) {
+    int nre = 0, npr = 0;
+    for (int s = 0; s < n_s; ++s) {
+      nre += K.r_co[lr + K.nr * s] != 0.0 ? 1 : 0;
+      npr += K.p_co[lr + K.nr * s] != 0.0 ? 1 : 0;
+    }
+    if (nre > KSIDE || npr > KSIDE) *flag = 0;
+  }
+  __syncthreads();
+  return *flag != 0;
+}
 
 }  // namespace streams

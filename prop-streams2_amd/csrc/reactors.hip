@@ -6,15 +6,15 @@
 // max(1,|w|).  Three forms of it (the `mixed` argument):
 //  0  the plain FP64 integrator, the yardstick of the other two: central-difference
 //     Jacobian over all N_S + 4 variables, FP64 Crout LU with implicit pivoting, and
-//     rosenbrock_rhs (:9249-9339) in the reference's own arithmetic forms (global NASA
-//     tables, reference-form kinetics from the packed records);
+//     rosenbrock_rhs (:9249-9339) in the reference's own arithmetic forms (reference-form
+//     kinetics from the packed records);
 //  1  mixed precision on the species block: one-sided species Jacobian, FP32 LU refined
 //     against the FP64 residual, fast-form kinetics and the NASA tables staged in LDS;
 //  2  form 1 with the LU in FP64 (no refinement): the like-for-like FP64 counterpart of 1,
 //     so that the difference between 1 and 2 is the precision of the factorisation alone.
 // Reactors have uneven stiffness, so a fixed
 // reactor-to-thread assignment would leave lanes idle behind the stiffest reactor of their
-// wave: instead every lane pulls its next reactor from a device-wide counter as soon as it
+// wave: instead every row of 16 lanes pulls its next reactor from a device-wide counter as soon as it
 // is done, and the grid is sized to the resident capacity of the GPU (persistent).
 #include "reactors_dev.h"
 
@@ -59,7 +59,6 @@ extern "C" int streams_reactor_batch(int n_s, int nbatch, double *w, double *tgu
   if (mixed != 0)
     return pressure != nullptr ? reactor_group_cp(n_s, indx_cp_l, indx_cp_r, A, ncu, wg_per_cu, st)
                                : reactor_group_cv(n_s, indx_cp_l, indx_cp_r, A, ncu, wg_per_cu, st);
-  if (indx_cp_r != 4 || (indx_cp_l != 0 && indx_cp_l != -2)) return STREAMS_E_OPTION;
-  if ((long)nbatch > (long)ncu * 256) return reactor_dispatch_wide(n_s, A, ncu, wg_per_cu, st);
-  return reactor_dispatch<false>(n_s, A, ncu, wg_per_cu, st);
+  return pressure != nullptr ? reactor_ref_cp(n_s, indx_cp_l, indx_cp_r, A, ncu, wg_per_cu, st)
+                             : reactor_ref_cv(n_s, indx_cp_l, indx_cp_r, A, ncu, wg_per_cu, st);
 }

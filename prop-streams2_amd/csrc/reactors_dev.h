@@ -1,7 +1,6 @@
 // reactors_dev.h — device code of the batched reactor integrator (streams_reactor_batch):
-// right-hand sides, the plain FP64 form's persistent kernel and its launchers.  Included by
-// reactors.hip (the narrow instance and the entry point), reactors_wide.hip (the wide
-// instance) and reactors_group_dev.h (the species-block forms).
+// arguments, right-hand sides of the species-block forms and the persistent grid.  Included by
+// reactors.hip (the entry point) and reactors_group_dev.h (the kernels).
 #pragma once
 #include <type_traits>
 
@@ -124,79 +123,6 @@ struct RosRhsPressure {
   }
 };
 
-// rosenbrock_rhs in the reference's arithmetic: constant volume (the reference's cell)
-template <int NS>
-struct RosRhsPackedRef {
-  const KinPacked &K;
-  const Thermo &th;
-  const double *mw;
-  double tol_iter_nr;
-  __device__ inline void operator()(double *wv, double &tg, double *rhs) const {
-    double yy[NS], conc[NS], acc[NS];
-#pragma unroll
-    for (int s = 0; s < NS; ++s) wv[s] = wv[s] > 0.0 ? wv[s] : 0.0;
-    double rho = wv[0];
-#pragma unroll
-    for (int s = 1; s < NS; ++s) rho = rho + wv[s];
-    const double ri = 1.0 / rho;
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      yy[s] = wv[s] * ri;
-      conc[s] = rho * yy[s] / mw[s];
-      acc[s] = 0.0;
-    }
-    const double uu = wv[NS] * ri, vv = wv[NS + 1] * ri, ww = wv[NS + 2] * ri;
-    const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
-    const double ee = wv[NS + 3] * ri - qq;
-    const double tt = temperature_from_e<NS>(ee, tg, th, tol_iter_nr, yy);
-    tg = tt;
-    chemistry_source_packed<NS, true>(K, tt, conc, acc, mw);
-#pragma unroll
-    for (int s = 0; s < NS; ++s) rhs[s] = -acc[s];
-#pragma unroll
-    for (int m = NS; m < NS + 4; ++m) rhs[m] = 0.0;
-  }
-};
-
-// The constant-pressure reactor in the same arithmetic: T from h by the e-inversion's
-// Newton iteration on the c_p tables (thh.cv_coeff holds cp_coeff), rho = p / (R T).
-template <int NS>
-struct RosRhsPressureRef {
-  const KinPacked &K;
-  const Thermo &thh;
-  const double *mw, *rgas;
-  double pres, tol_iter_nr;
-  __device__ inline void operator()(double *wv, double &tg, double *rhs) const {
-    double yy[NS], conc[NS], acc[NS];
-#pragma unroll
-    for (int s = 0; s < NS; ++s) wv[s] = wv[s] > 0.0 ? wv[s] : 0.0;
-    double ysum = wv[0];
-#pragma unroll
-    for (int s = 1; s < NS; ++s) ysum = ysum + wv[s];
-    const double yi = 1.0 / ysum;
-    double rmix = 0.0;
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      yy[s] = wv[s] * yi;
-      rmix = rmix + rgas[s] * yy[s];
-    }
-    const double tt = temperature_from_e<NS>(wv[NS + 3], tg, thh, tol_iter_nr, yy);
-    tg = tt;
-    const double rho = pres / (rmix * tt);
-    const double ri = 1.0 / rho;
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      conc[s] = rho * yy[s] / mw[s];
-      acc[s] = 0.0;
-    }
-    chemistry_source_packed<NS, true>(K, tt, conc, acc, mw);
-#pragma unroll
-    for (int s = 0; s < NS; ++s) rhs[s] = -acc[s] * ri;
-#pragma unroll
-    for (int m = NS; m < NS + 4; ++m) rhs[m] = 0.0;
-  }
-};
-
 struct ReactorArgs {
   double *w, *tg;                 // w[m * nbatch + b] (SoA), T guess / result
   const double *dttry, *time_end; // per reactor
@@ -210,66 +136,6 @@ struct ReactorArgs {
   KinPacked K;
   Thermo th;
 };
-
-template <int NS, class Rhs>
-__device__ inline void integrate_one(const Rhs &f, const ReactorArgs &A, unsigned r) {
-  constexpr int NV = NS + 4;
-  const long nb = A.nbatch;
-  double wv[NV];
-#pragma unroll
-  for (int m = 0; m < NV; ++m) wv[m] = A.w[(long)m * nb + r];
-  double tg = A.tg[r];
-  RosStats st;
-  double t0 = 0.0, dt0 = A.dttry[r];
-  if (A.t_done) {
-    st.resume = true;
-    t0 = A.t_done[r];
-    if (A.dt_next[r] > 0.0) dt0 = A.dt_next[r];
-    if (t0 >= A.time_end[r]) {                        // finished earlier: nothing to do
-      if (A.nacc) A.nacc[r] = 0;
-      if (A.nrej) A.nrej[r] = 0;
-      return;
-    }
-  }
-  rosenbrock_cell_f<NS>(f, wv, tg, dt0, t0, A.time_end[r], A.maxsteps, A.maxtry, A.tol, st);
-#pragma unroll
-  for (int m = 0; m < NV; ++m) A.w[(long)m * nb + r] = wv[m];
-  A.tg[r] = tg;
-  if (A.nacc) A.nacc[r] = st.nacc;
-  if (A.nrej) A.nrej[r] = st.nrej;
-  if (A.t_done) {
-    A.t_done[r] = st.done ? A.time_end[r] : st.t_end;
-    A.dt_next[r] = st.dt_next;
-  }
-}
-
-// Waves per SIMD the compiler budgets registers for in the plain FP64 form, one lane per
-// reactor.  It spills (the per-lane Jacobian, its factors and the four stage vectors do not
-// fit).  A batch larger than the GPU holds at one wave per SIMD (CUs x 256 lanes) runs the
-// WIDE instance: more resident waves then hide the spill and table latencies better than
-// fewer, larger register files.  A smaller batch cannot fill the extra waves, and each lane
-// is faster at one wave.  The two instances are compiled in separate translation units
-// (reactors.hip, reactors_wide.hip): device code that both called would get one register
-// budget for both.
-template <int NS, bool CP, bool WIDE>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WIDE ? 2 : 1)))
-reactor_kernel(ReactorArgs A) {
-  // reads the NASA tables from global memory in the reference's forms
-  Thermo thh = A.th;
-  thh.cv_coeff = A.th.cp_coeff;
-  const long nb = A.nbatch;
-  for (;;) {
-    const unsigned r = atomicAdd(A.next, 1u);
-    if ((long)r >= nb) break;
-    if (CP) {
-      const RosRhsPressureRef<NS> f{A.K, thh, A.mw, A.rgas, A.pressure[r], A.tol_iter_nr};
-      integrate_one<NS>(f, A, r);
-    } else {
-      const RosRhsPackedRef<NS> f{A.K, A.th, A.mw, A.tol_iter_nr};
-      integrate_one<NS>(f, A, r);
-    }
-  }
-}
 
 // Persistent grid: wg_per_cu workgroups per CU (default 4, at least the resident capacity
 // of these register-heavy kernels), never more than the batch needs at `per_wg` reactors a
@@ -295,22 +161,10 @@ inline int reactor_grid(int ncu, int wg_per_cu, int min_per_cu, int per_wg, long
   return (int)(g < need ? g : need);
 }
 
-// Launch of one instance of the plain FP64 form (instantiated in one translation unit per
-// instance).
-template <bool WIDE>
-int reactor_dispatch(int n_s, const ReactorArgs &A, int ncu, int wg_per_cu, hipStream_t st) {
-  const int g = reactor_grid(ncu, wg_per_cu, WIDE ? 2 : 1, 256, A.nbatch);
-  if (g <= 0) return STREAMS_E_DIMS;
-  if (A.pressure != nullptr) {
-    STREAMS_DISPATCH_NS(n_s, (reactor_kernel<NS, true, WIDE><<<g, 256, 0, st>>>(A)));
-  } else {
-    STREAMS_DISPATCH_NS(n_s, (reactor_kernel<NS, false, WIDE><<<g, 256, 0, st>>>(A)));
-  }
-  return hip_status();
-}
-
-// the wide instance, compiled in reactors_wide.hip
-int reactor_dispatch_wide(int n_s, const ReactorArgs &A, int ncu, int wg_per_cu, hipStream_t st);
+// the plain FP64 form (reactors_ref_dev.h), compiled in reactors_ref.hip (constant volume) and
+// reactors_ref_cp.hip (constant pressure)
+int reactor_ref_cv(int n_s, int indx_cp_l, int indx_cp_r, const ReactorArgs &A, int ncu, int wg_per_cu, hipStream_t st);
+int reactor_ref_cp(int n_s, int indx_cp_l, int indx_cp_r, const ReactorArgs &A, int ncu, int wg_per_cu, hipStream_t st);
 
 // the species-block forms (reactors_group_dev.h), compiled in reactors_group.hip (constant
 // volume) and reactors_group_cp.hip (constant pressure)

@@ -55,12 +55,12 @@ __device__ inline double row_shuffle(double v, int src) { return __shfl(v, src, 
 
 // Crout LU with implicit partial pivoting (ludcmp), row l in lane l: the right-looking order
 // subtracts the same products from each element in the same order.  perm returns the lane
-// whose right-hand side component this row's equation takes.
+// whose right-hand side component this row's equation takes; amax: largest magnitude of the
+// row's elements beside the N columns.
 template <int N, class T>
-__device__ inline void row_ludcmp(T *a, int l, int &perm) {
+__device__ inline void row_ludcmp(T *a, int l, int &perm, T amax = 0) {
   const T tiny = (T)1.5e-16;
   perm = l;
-  T amax = 0;
   static_for<0, N>([&](auto J) { amax = fabs(a[J]) > amax ? fabs(a[J]) : amax; });
   const unsigned long low = __ballot(l < N && amax < tiny);
   const int sh = (int)(threadIdx.x & 48);

@@ -15,8 +15,8 @@ namespace streams {
 // face in registers (nx*nz*ny/16 threads, whose enthalpies and loads ran one after the other)
 // or exchanging faces through LDS.  The faces of a cell share its own values; the arithmetic of
 // a face is the reference's.  96x72x60 cells, 9 species: x 0.128 -> 0.054 ms, y 0.505 -> 0.061, z
-// 0.505 -> 0.085; bounded by the loads of three cells and the six enthalpies of a species.  LO: NASA form of the tables staged in LDS, 99: any other form, from
-// global memory.
+// 0.505 -> 0.085; bounded by the loads of three cells and the enthalpies of a species there.  LO:
+// NASA form of the tables staged in LDS, 99: any other form, from global memory.
 template <int NS, int DIR, int LO>
 __global__ void __launch_bounds__(256) visc_cell_kernel(Box b, ViscArgs A, unsigned ncells) {
   using X = Idx<NS>;
@@ -43,7 +43,8 @@ __global__ void __launch_bounds__(256) visc_cell_kernel(Box b, ViscArgs A, unsig
   double T[2];
   const double tc = at(0, X::J_T);
   {
-    const double uc = at(0, X::J_U), vc = at(0, X::J_V), wc = at(0, X::J_W), mu = at(0, X::J_MU), kc = at(0, X::J_K_COND);
+    const double uc = at(0, X::J_U), vc = at(0, X::J_V), wc = at(0, X::J_W);
+    const double mu = at(0, X::J_MU), kc = at(0, X::J_K_COND);
     const double qc = 0.5 * (uc * uc + vc * vc + wc * wc);
     double sx = 0.0, sy = 0.0, sz = 0.0, sq = 0.0;
 #pragma unroll

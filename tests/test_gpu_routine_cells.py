@@ -49,8 +49,8 @@ def _fl(pkg, oracle, tb, shape, ng, num, stage, bctags=(0,) * 6, force=None, see
     ((7, 8, 9), 3, 6, -1, (2, 2, 2, 2, 2, 2), [0, 1, 1, 1, 0, 1]),
 ])
 def test_euler_without_sensor(pkg, oracle, h2_tables, d, shape, ng, order, nkeep, bc, force):
-    num = pkg.solver.Numerics(ep_order=order, visc_order=order, nkeep=nkeep, sensor_threshold=2.0, weno_scheme=min(ng, 3),
-                              correct_bound_ord=int(bc[0] != 0))
+    num = pkg.solver.Numerics(ep_order=order, visc_order=order, nkeep=nkeep, sensor_threshold=2.0,
+                              weno_scheme=min(ng, 3), correct_bound_ord=int(bc[0] != 0))
     err = _fl(pkg, oracle, h2_tables, shape, ng, num, lambda s: s.euler(d), bc, force)
     assert err.max() < TOL, err
 
