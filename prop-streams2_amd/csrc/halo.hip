@@ -12,18 +12,21 @@
 namespace streams {
 
 // axis 0: (i in 1..ng, j in 1..ny, k in 1..nz); axis 1: (i 1..nx, j 1..ng, k 1..nz);
-// axis 2: (i 1..nx, j 1..ny, k 1..ng).  The flat index covers side, variable, slab.
+// axis 2: (i 1..nx, j 1..ny, k 1..ng).  The flat index covers slab, side, variable; on an axis
+// shorter than ng it covers the lines across the slabs (extent 1 along the axis) and variables.
+template <class I>
 struct Slab {
-  int ax, nv;
-  int e0, e1, e2;  // extents of the slab in i, j, k
-  __device__ inline void decode(long t, int &side, int &m, int &a, int &bq, int &c) const {
-    a = 1 + (int)(t % e0); t /= e0;
-    bq = 1 + (int)(t % e1); t /= e1;
-    c = 1 + (int)(t % e2); t /= e2;
-    m = (int)(t % nv); t /= nv;
-    side = (int)t;
-  }
+  I n;                      // threads of this axis
+  unsigned blocks;
+  int e0, e1, e2;           // extents in i, j, k
+  bool line;
 };
+template <class I>
+struct SwapPlan {
+  Slab<I> ax[3];
+};
+
+constexpr int NG_LINE = 8;  // deepest ghost layer a line keeps in registers
 
 __device__ inline void slab_src_dst(const Box &b, int ax, int side, int a, int bq, int c, long &src,
                                     long &dst) {
@@ -41,48 +44,72 @@ __device__ inline void slab_src_dst(const Box &b, int ax, int side, int a, int b
   }
 }
 
-__global__ void __launch_bounds__(256) swap_direct_kernel(Box b, Slab s, long n, double *__restrict__ w) {
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  int side, m, a, bq, c;
-  s.decode(t, side, m, a, bq, c);
+// All periodic axes in one launch, a range of workgroups per axis: a launch takes about 4 us on
+// this GPU, as long as its copies in a small box (19x14x11 cells: three launches 10.5 us -> one of
+// 4).  On an axis shorter than ng the sources lie in ghosts that are written as well, but only in
+// those of the same line: a thread reads its line's sources before it writes any, which takes the
+// place of a staging buffer's allocation and two more launches.
+template <class I>
+__global__ void __launch_bounds__(256) swap_kernel(Box b, SwapPlan<I> plan, double *__restrict__ w) {
+  unsigned blk = blockIdx.x;
+  int ax = 0;
+  if (blk >= plan.ax[0].blocks) { blk -= plan.ax[0].blocks; ax = 1; }
+  if (ax == 1 && blk >= plan.ax[1].blocks) { blk -= plan.ax[1].blocks; ax = 2; }
+  const Slab<I> s = plan.ax[ax];
+  I t = (I)blk * 256 + threadIdx.x;
+  if (t >= s.n) return;
+  const int a = 1 + (int)(t % s.e0); t /= s.e0;
+  const int bq = 1 + (int)(t % s.e1); t /= s.e1;
+  const int c = 1 + (int)(t % s.e2); t /= s.e2;
   long src, dst;
-  slab_src_dst(b, s.ax, side, a, bq, c, src, dst);
-  const long ps = b.pstride() * m;
-  w[dst + ps] = w[src + ps];
+  if (s.line && b.ng > NG_LINE) {
+    // deeper: in place, each side from the end that its sources are written last
+    double *v = w + b.pstride() * (long)t;
+    for (int side = 0; side < 2; ++side)
+      for (int q = 0; q < b.ng; ++q) {
+        const int l = side == 0 ? 1 + q : b.ng - q;
+        slab_src_dst(b, ax, side, ax == 0 ? l : a, ax == 1 ? l : bq, ax == 2 ? l : c, src, dst);
+        v[dst] = v[src];
+      }
+  } else if (s.line) {
+    double *v = w + b.pstride() * (long)t;
+    double x[2][NG_LINE];
+#pragma unroll
+    for (int side = 0; side < 2; ++side)
+#pragma unroll
+      for (int l = 0; l < NG_LINE; ++l)
+        if (l < b.ng) {
+          slab_src_dst(b, ax, side, ax == 0 ? 1 + l : a, ax == 1 ? 1 + l : bq, ax == 2 ? 1 + l : c, src, dst);
+          x[side][l] = v[src];
+        }
+#pragma unroll
+    for (int side = 0; side < 2; ++side)
+#pragma unroll
+      for (int l = 0; l < NG_LINE; ++l)
+        if (l < b.ng) {
+          slab_src_dst(b, ax, side, ax == 0 ? 1 + l : a, ax == 1 ? 1 + l : bq, ax == 2 ? 1 + l : c, src, dst);
+          v[dst] = x[side][l];
+        }
+  } else {
+    slab_src_dst(b, ax, (int)(t & 1), a, bq, c, src, dst);
+    const long ps = b.pstride() * (long)(t >> 1);
+    w[dst + ps] = w[src + ps];
+  }
 }
 
-__global__ void __launch_bounds__(256) swap_pack_kernel(Box b, Slab s, long n, const double *__restrict__ w,
-                                                        double *__restrict__ buf) {
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  int side, m, a, bq, c;
-  s.decode(t, side, m, a, bq, c);
-  long src, dst;
-  slab_src_dst(b, s.ax, side, a, bq, c, src, dst);
-  buf[t] = w[src + b.pstride() * m];
-}
-
-__global__ void __launch_bounds__(256) swap_unpack_kernel(Box b, Slab s, long n, double *__restrict__ w,
-                                                          const double *__restrict__ buf) {
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  int side, m, a, bq, c;
-  s.decode(t, side, m, a, bq, c);
-  long src, dst;
-  slab_src_dst(b, s.ax, side, a, bq, c, src, dst);
-  w[dst + b.pstride() * m] = buf[t];
-}
-
-// bcextr_var_cuf / bcextr_cuf: zero-order extrapolation of face ilat (1..6)
-__global__ void __launch_bounds__(256) extr_kernel(Box b, int ilat, int nv, long n, double *__restrict__ w) {
+// bcextr_var_cuf / bcextr_cuf: zero-order extrapolation of the faces first..last (1..6) of
+// nv variables, a row of workgroups (blockIdx.y) per face; sources are interior points, so the
+// faces are independent.
+__global__ void __launch_bounds__(256) extr_kernel(Box b, int first, int nv, double *__restrict__ w) {
+  const int ilat = first + (int)blockIdx.y;
+  const int e0 = (ilat <= 2) ? b.ny : b.nx;
+  const int e1 = (ilat <= 4) ? b.nz : b.ny;
+  const long n = (long)b.ng * e0 * e1 * nv;
   long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
   int l, a, c, m;
   // flat index: l fastest, then the two face coordinates, then the variable
   l = 1 + (int)(t % b.ng); long r = t / b.ng;
-  int e0 = (ilat <= 2) ? b.ny : b.nx;
-  int e1 = (ilat <= 4) ? b.nz : b.ny;
   a = 1 + (int)(r % e0); r /= e0;
   c = 1 + (int)(r % e1); r /= e1;
   m = (int)r;
@@ -125,33 +152,37 @@ __global__ void __launch_bounds__(256) wall_ad_kernel(Box b, int ilat, int ns, l
   (void)nv;
 }
 
-int extr_faces(const Box &b, int ilat, int nv, double *w, hipStream_t st) {
-  int e0 = (ilat <= 2) ? b.ny : b.nx;
-  int e1 = (ilat <= 4) ? b.nz : b.ny;
-  long n = (long)b.ng * e0 * e1 * nv;
+int extr_faces(const Box &b, int first, int last, int nv, double *w, hipStream_t st) {
+  long n = 0;                                        // points of the largest face
+  for (int ilat = first; ilat <= last; ++ilat) {
+    const long f = (long)b.ng * (ilat <= 2 ? b.ny : b.nx) * (ilat <= 4 ? b.nz : b.ny) * nv;
+    n = f > n ? f : n;
+  }
   if (n <= 0) return 0;
-  extr_kernel<<<blocks_for(n, 256), 256, 0, st>>>(b, ilat, nv, n, w);
+  extr_kernel<<<dim3(blocks_for(n, 256), last - first + 1), 256, 0, st>>>(b, first, nv, w);
   return hip_status();
 }
 
-int swap_axis(const Box &b, int ax, int nv, double *w, hipStream_t st) {
-  int n_ax = ax == 0 ? b.nx : ax == 1 ? b.ny : b.nz;
-  Slab s{ax, nv, ax == 0 ? b.ng : b.nx, ax == 1 ? b.ng : b.ny, ax == 2 ? b.ng : b.nz};
-  long n = 2L * s.e0 * s.e1 * s.e2 * nv;
-  if (n <= 0) return 0;
-  if (n_ax >= b.ng) {
-    swap_direct_kernel<<<blocks_for(n, 256), 256, 0, st>>>(b, s, n, w);
-  } else {
-    // stream-ordered staging: calls on different streams each get their own buffer
-    double *buf = nullptr;
-    if (hipMallocAsync((void **)&buf, (size_t)n * sizeof(double), st) != hipSuccess) return STREAMS_E_NOMEM;
-    swap_pack_kernel<<<blocks_for(n, 256), 256, 0, st>>>(b, s, n, w, buf);
-    swap_unpack_kernel<<<blocks_for(n, 256), 256, 0, st>>>(b, s, n, w, buf);
-    const int rc = hip_status();
-    const hipError_t e = hipFreeAsync(buf, st);
-    if (rc) return rc;
-    return e == hipSuccess ? 0 : (int)e;
+// 64-bit point indices only where a slab holds more points than 32 bits count
+template <class I>
+int swap_launch(const Box &b, const int *periodic, int nv, double *w, hipStream_t st) {
+  SwapPlan<I> plan{};
+  unsigned g = 0;
+  const int n[3] = {b.nx, b.ny, b.nz};
+  for (int ax = 0; ax < 3; ++ax) {
+    Slab<I> &s = plan.ax[ax];
+    if (!periodic[ax]) continue;
+    s.line = n[ax] < b.ng;
+    const int depth = s.line ? 1 : b.ng;
+    s.e0 = ax == 0 ? depth : b.nx;
+    s.e1 = ax == 1 ? depth : b.ny;
+    s.e2 = ax == 2 ? depth : b.nz;
+    s.n = (I)s.e0 * s.e1 * s.e2 * nv * (s.line ? 1 : 2);
+    s.blocks = blocks_for((long)s.n, 256);
+    g += s.blocks;
   }
+  if (g == 0) return 0;
+  swap_kernel<I><<<g, 256, 0, st>>>(b, plan, w);
   return hip_status();
 }
 
@@ -166,28 +197,21 @@ extern "C" int streams_bcswap(int nx, int ny, int nz, int ng, int nv, double *w,
   hipStream_t st = as_stream(stream);
   // The reference packs all six slabs before unpacking any.  Sources of one axis never lie
   // in the ghost slabs of another axis (their tangential indices are interior), so the
-  // axes are independent; only the short-axis self-overlap needs staging.
-  for (int ax = 0; ax < 3; ++ax) {
-    if (!periodic[ax]) continue;
-    int rc = swap_axis(b, ax, nv, w, st);
-    if (rc) return rc;
-  }
-  return 0;
+  // axes are independent.
+  const long most = 2L * ng * nv;
+  const bool wide = most * ny * nz > 0xfff00000l || most * nx * nz > 0xfff00000l || most * nx * ny > 0xfff00000l;
+  return wide ? swap_launch<unsigned long>(b, periodic, nv, w, st) : swap_launch<unsigned>(b, periodic, nv, w, st);
 }
 
 extern "C" int streams_bcextr_var(int nx, int ny, int nz, int ng, double *w_var, void *stream) {
   Box b{nx, ny, nz, ng};
-  for (int ilat = 1; ilat <= 6; ++ilat) {
-    int rc = extr_faces(b, ilat, 1, w_var, as_stream(stream));
-    if (rc) return rc;
-  }
-  return 0;
+  return extr_faces(b, 1, 6, 1, w_var, as_stream(stream));
 }
 
 extern "C" int streams_bcextr(int ilat, int nx, int ny, int nz, int ng, int nv, double *w, void *stream) {
   if (ilat < 1 || ilat > 6) return STREAMS_E_DIMS;
   Box b{nx, ny, nz, ng};
-  return extr_faces(b, ilat, nv, w, as_stream(stream));
+  return extr_faces(b, ilat, ilat, nv, w, as_stream(stream));
 }
 
 extern "C" int streams_bcwall_ad(int n_s, int ilat, int nx, int ny, int nz, int ng, double *w, void *stream) {
