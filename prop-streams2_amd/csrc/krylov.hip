@@ -1,7 +1,7 @@
 // krylov.hip — the Rosenbrock–Krylov integrator of the stiff chemistry (FP64).
 //
-// One thread per interior cell restates rosenbrock_krylov_kernel
-// (kernels_gpu.F90:10360-10611): a 4-stage ROK method whose linear algebra lives in a
+// One thread per interior cell (half a wave in small fields: krylov_rows.hip) restates
+// rosenbrock_krylov_kernel (kernels_gpu.F90:10360-10611): a 4-stage ROK method whose linear algebra lives in a
 // Krylov space of at most KM = 4 vectors (M_max, index_define.h:27), rebuilt by Arnoldi
 // (arnoldi, :10664-10792) on one-sided finite-difference Jacobian-vector products
 // (rosenbrock_krylov_jacobian, :10613-10662) for every attempted step.  Only cells with a
@@ -9,6 +9,7 @@
 // side is rosenbrock_krylov_rhs (:10794-10976), which is rosenbrock_rhs's arithmetic on a
 // copy of the state with the temperature guess passed by value.
 #include "chem_common.h"
+#include "kinpack.h"
 
 namespace streams {
 
@@ -217,14 +218,19 @@ __device__ int krylov_cell(const Kin &K, const Thermo &th, double tol_iter_nr, d
 
 // 2 waves per SIMD (the compiler's own choice is 1, with 2.8-3.7 KB of per-lane spills):
 // the extra resident wave hides the spill latency (one integration of a 128^3 box at 1500 K,
-// 25.7 -> 22.2 ms; 3 waves: 26.1 ms; bit-identical)
+// 25.7 -> 22.2 ms; 3 waves: 26.1 ms; bit-identical).  rows: krylov_rows was launched and takes the
+// call if every side of the reactions fits its records.
 template <int NS>
 __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) krylov_kernel(Box b, double *__restrict__ w, const double *__restrict__ w_aux,
                                                      Kin K, Thermo th, double tol_iter_nr, double dttry,
                                                      double time_start, double time_end, int maxsteps,
-                                                     const double *__restrict__ fl_sav, Pasr pasr) {
+                                                     const double *__restrict__ fl_sav, Pasr pasr, bool rows) {
   using X = Idx<NS>;
   constexpr int NV = NS + 4;
+  if (rows) {
+    __shared__ int flag;
+    if (sides_fit(NS, K, &flag)) return;
+  }
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= b.fstride()) return;
   const int i = 1 + (int)(t % b.nx);
@@ -243,6 +249,15 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) k
                   fl_sav ? fls : nullptr, tau_k);
   for (int m = 0; m < NV; ++m) w[pt + ps * m] = vec[m];
 }
+
+int krylov_rows(int n_s, const Box &b, double *w, const double *w_aux, const Kin &K, const Thermo &th,
+                double tol_iter_nr, double dttry, double time_start, double time_end, int maxsteps,
+                const double *fl_sav, const Pasr &pasr, hipStream_t st);
+// Cells up to which half a wave per cell is faster (random states, one interval of 1e-8 s, 9
+// species): 800 cells 939 -> 236 ms, 8000 cells 1079 -> 774; 4096 cells are in flight at once, above
+// some 8000 the repeated scalar work of the 32 lanes costs what the shorter chain gains.
+constexpr long KROWS_CELLS = 8192;
+constexpr long KROWS_LDS = 36 * 1024;        // bytes of records at most
 
 }  // namespace streams
 
@@ -272,8 +287,15 @@ extern "C" int streams_rosenbrock_krylov(int n_s, int nv, int nv_aux, int nx, in
         nreactions, num_t_tab, t_min_tab, dt_tab, r_univ};
   Thermo th{cv_coeff, nullptr, trange, nsetcv, indx_cp_l, indx_cp_r};
   const double *fls = simpler_splitting == 1 ? fl_sav : nullptr;
-  STREAMS_DISPATCH_NS(n_s, (krylov_kernel<NS><<<blocks_for(n, 128), 128, 0, as_stream(stream)>>>(
+  const bool rows = (indx_cp_l == 0 || indx_cp_l == -2) && indx_cp_r == 4 && (long)nreactions * KREC * 8 <= KROWS_LDS &&
+                    n <= KROWS_CELLS;
+  hipStream_t st = as_stream(stream);
+  if (rows) {
+    const int rc = krylov_rows(n_s, b, w, w_aux, K, th, tol_iter_nr, dttry, time_start, time_end, maxsteps, fls, pasr, st);
+    if (rc) return rc;
+  }
+  STREAMS_DISPATCH_NS(n_s, (krylov_kernel<NS><<<blocks_for(n, 128), 128, 0, st>>>(
                                 b, w, w_aux, K, th, tol_iter_nr, dttry, time_start, time_end, maxsteps, fls,
-                                pasr)));
+                                pasr, rows)));
   return hip_status();
 }

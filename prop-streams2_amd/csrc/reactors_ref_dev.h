@@ -35,6 +35,29 @@ struct RefArgs {
   unsigned ncells;
 };
 
+// Rate of progress of reaction r in the reference's forms at the concentrations c (LDS); d gets
+// p - r of the species, NaN for those that take no part.
+template <int NS>
+__device__ inline double row_reaction(const KinPacked &K, const double *pack, int r, double tt, double Rtti, double dtt,
+                                      int itt, const double *c, double *d) {
+  const double *R = pack + KREC * r;
+  const int *I = (const int *)R;
+  const double q = reaction_progress<NS, true>(R, I, K.kc_tab + (itt - 1) + ((long)K.num_t_tab + 1) * r, tt, 0.0, Rtti,
+                                               dtt, [&](int s) { return c[s]; }, [&](int s) { return c[s]; });
+#pragma unroll
+  for (int s = 0; s < GROW; ++s) d[s] = __builtin_nan("");
+#pragma unroll
+  for (int e = 0; e < KSIDE; ++e)
+    if (e < I[KI_NRE]) d[I[KI_RE + e]] = -R[KD_REX + e];
+#pragma unroll
+  for (int e = 0; e < KSIDE; ++e)
+    if (e < I[KI_NPR]) {
+      const double v = d[I[KI_PR + e]];
+      d[I[KI_PR + e]] = v == v ? R[KD_PEX + e] + v : R[KD_PEX + e];
+    }
+  return q;
+}
+
 // row_source in the reference's forms: acc_s -= ((p - r) q) W_s over the species of each reaction.
 // dn: 16 x 16 doubles, p - r of species s in reaction k, NaN when it takes no part.
 template <int NS>
@@ -46,29 +69,13 @@ __device__ inline double row_source_ref(const KinPacked &K, const double *pack, 
   itt = itt > K.num_t_tab ? K.num_t_tab : itt;
   const double ttleft = (itt - 1) * K.dt_tab + K.t_min_tab;
   const double dtt = (tt - ttleft) / K.dt_tab;
-  const long ntab = (long)K.num_t_tab + 1;
   double acc = 0.0;
   cl[l] = c;
   for (int r0 = 0; r0 < K.nr; r0 += GROW) {
     const int r = r0 + l;
     row_sync();
     if (r < K.nr) {
-      const double *R = pack + KREC * r;
-      const int *I = (const int *)R;
-      ql[l] = reaction_progress<NS, true>(R, I, K.kc_tab + (itt - 1) + ntab * r, tt, 0.0, Rtti, dtt,
-                                          [&](int s) { return cl[s]; }, [&](int s) { return cl[s]; });
-      double *d = dn + GROW * l;
-#pragma unroll
-      for (int s = 0; s < GROW; ++s) d[s] = __builtin_nan("");
-#pragma unroll
-      for (int e = 0; e < KSIDE; ++e)
-        if (e < I[KI_NRE]) d[I[KI_RE + e]] = -R[KD_REX + e];
-#pragma unroll
-      for (int e = 0; e < KSIDE; ++e)
-        if (e < I[KI_NPR]) {
-          const double v = d[I[KI_PR + e]];
-          d[I[KI_PR + e]] = v == v ? R[KD_PEX + e] + v : R[KD_PEX + e];
-        }
+      ql[l] = row_reaction<NS>(K, pack, r, tt, Rtti, dtt, itt, cl, dn + GROW * l);
     }
     row_sync();
     const int n = K.nr - r0 < GROW ? K.nr - r0 : GROW;
