@@ -68,6 +68,8 @@ class TimedBackend:
         if name == "rhs_sweep":
             key = f"rhs_sweep_{args[0]}"
             tag = key + ("_set" if args[-5] == 2 else "")
+        elif name == "rhs_cells":
+            key, tag = name, (name + "_next" if args[-4] else name)         # the next init_flux folded in
         elif name == "rhs_finish_next":
             key, tag = "rhs_finish", name
         elif name == "eval_aux2":
@@ -96,6 +98,7 @@ class TimedBackend:
 
 # GPU kernels each timed entry point launches (the fused path, KEEP central, sixth order)
 ENTRY_KERNELS = {
+    "rhs_cells": ["cell_momentum_kernel<NS, 3>", "cell_species_kernel<NS, 3>", "finish_species_kernel<NS>"],
     "rhs_finish": ["finish_species_kernel<NS>", "finish_mom_kernel<NS, 3>"],
     "rhs_sweep_1": ["sweep_kernel<NS, 1, 0, 3>"],
     "rhs_sweep_2": ["sweep_kernel<NS, 2, 0, 3>"],
@@ -397,7 +400,7 @@ def main():
     be = pkg.solver.HipBackend("cuda:0")
     entries = ["eval_aux", "eval_aux2", "euler_x", "euler_y", "euler_z", "visflx_x", "visflx_y", "visflx_z",
                "visflx_reduced", "compute_chemistry", "init_flux", "update_flux", "update_field", "bcswap",
-               "bcextr_var", "rhs_sweep_1", "rhs_sweep_2", "rhs_sweep_3", "rhs_finish"]
+               "bcextr_var", "rhs_sweep_1", "rhs_sweep_2", "rhs_sweep_3", "rhs_finish", "rhs_cells"]
     tbe = TimedBackend(be, entries)
     s = pkg.solver.Solver(tbe, tables, n, n, n, 3, [info["length"]] * 3, rho0=info["rho0"], u0=info["u_rms"])
     s.set_state(w, tg)

@@ -94,7 +94,7 @@ __global__ void __launch_bounds__(256) chemistry_kernel(Box b, double *__restric
 
 // workgroups of chemistry_kernel: each packs the tables once, so no more than fill the GPU
 constexpr long CHEM_BLOCKS = 1024;
-constexpr long CHEM_LDS = 64 * 1024;         // bytes of records at most
+constexpr long CHEM_LDS = 48 * 1024;         // bytes of records at most, beside up to 8 KB of NASA tables
 
 template <int NS, int LO>
 void chemistry_launch(const Box &b, double *w, double *w_aux, double *fl, const Kin &K, const Thermo &th, double tol,

@@ -19,6 +19,9 @@ its roofline fraction.  Counts per point, N_S species, NV = N_S + 4:
   rhs_finish        interior       read 5 + N_S + 2 (u, v, w, mu, div/3, rho, T, Y),
                                    fl, fln, w read+write 6 NV
   rhs_finish_next   interior       the same without the fl store: 5 NV
+  rhs_cells         interior       read 2 N_S + 10 (Y, rho D, rho, u, v, w, h, p, T, mu, k, div/3)
+                                   and fl or fln, w read+write, write fl and fln: 5 NV
+  rhs_cells_next    interior       the same without the fl store: 4 NV
 """
 from __future__ import annotations
 
@@ -42,6 +45,8 @@ def per_point_doubles(name: str, ns: int) -> int:
         "rhs_sweep_1_set": (ns + 6) + (ns + 3) + nv,
         "rhs_finish": 7 + ns + 6 * nv,
         "rhs_finish_next": 7 + ns + 5 * nv,
+        "rhs_cells": 2 * ns + 10 + 5 * nv,
+        "rhs_cells_next": 2 * ns + 10 + 4 * nv,
     }
     return table.get(name, 0)
 

@@ -75,7 +75,8 @@ def test_viscous_faces(pkg, oracle, shape, mech, general):
 
 @pytest.mark.parametrize("shape,mech,change", [((37, 5, 3), "h2", "none"), ((64, 2, 2), "keromnes", "none"),
                                                ((5, 7, 33), "h2", "general"), ((9, 8, 7), "h2", "five"),
-                                               ((9, 8, 7), "h2", "many"), ((150, 60, 40), "h2", "none")])
+                                               ((9, 8, 7), "h2", "many"), ((9, 8, 7), "h2", "three"),
+                                               ((150, 60, 40), "h2", "none")])
 def test_chemistry_tables(pkg, oracle, shape, mech, change):
     """(150, 60, 40): more cells than the grid's threads, so a workgroup takes several rounds."""
     from test_gpu_cells import _tables
@@ -87,8 +88,8 @@ def test_chemistry_tables(pkg, oracle, shape, mech, change):
         r[0] = 0.0
         r[0, :5] = (1.0, 0.5, 2.0, 1.0, 0.25)
         tb = dataclasses.replace(tb, r_coeffs=r)
-    elif change == "many":
-        rep = 110 // tb.nreactions + 1
+    elif change in ("many", "three"):            # beyond the local memory, and most of it
+        rep = 6 if change == "many" else 3
         cat = lambda a, ax=0: np.concatenate([np.asarray(a)] * rep, axis=ax)  # noqa: E731
         kc = np.asarray(tb.kc_tab)
         rows = {f: cat(getattr(tb, f)) for f in ("reac_ty", "isRev", "arr_a", "arr_b", "arr_ea", "falloff_coeffs",
