@@ -34,8 +34,9 @@ struct CellArgs {
   int init, fold;
 };
 
-// Tiles of TX x TY x TZ cells, one per thread, y tiles of a band fastest, then z, then x, then
-// the next band; one contiguous range of tiles per XCD.
+// Tiles of TX x TY x TZ cells, one per thread, x fastest, then the y tiles of a band, then z, then the
+// next band; one contiguous range of tiles per XCD.  Whole rows first, because a row of 38 cells
+// touches up to twice the 128-byte lines of its 32: 256^3 8.51 -> 8.25 ms a call.
 constexpr int TX = 32, TY = 4, TZ = 2, YBAND = 8;
 struct CellTiles {
   int nxt, nzt, yb;           // tiles along x and z, y tiles of a band
@@ -52,12 +53,12 @@ inline bool cell_tiles(const Box &b, CellTiles &r) {
 }
 // First cell of this workgroup's tile (it may lie past ny in the last band).
 __device__ inline void tile_origin(const CellTiles &r, unsigned tile, int &i0, int &j0, int &k0) {
+  i0 = 1 + TX * (int)(tile % r.nxt);
+  tile /= r.nxt;
   const int y = (int)(tile % r.yb);
   tile /= r.yb;
   k0 = 1 + TZ * (int)(tile % r.nzt);
-  tile /= r.nzt;
-  i0 = 1 + TX * (int)(tile % r.nxt);
-  j0 = 1 + TY * ((int)(tile / r.nxt) * r.yb + y);
+  j0 = 1 + TY * ((int)(tile / r.nzt) * r.yb + y);
 }
 
 // A tile of one plane with its star of W cells on each side in LDS: [z][y][x] with the
