@@ -56,6 +56,10 @@ extern "C" int streams_reactor_batch(int n_s, int nbatch, double *w, double *tgu
                 Thermo{cv_coeff, cp_coeff, trange, nsetcv, indx_cp_l, indx_cp_r}};
   zero_counter_kernel<<<1, 1, 0, st>>>(work);
   const int ncu = device_cus();
+  if (mixed == 2 && pressure == nullptr && nbatch >= LANES_FROM && nbatch < (1 << 30)) {
+    const int rc = reactor_lanes(n_s, indx_cp_l, indx_cp_r, A, ncu, wg_per_cu, st);
+    if (rc) return rc;                               // rows find the counter past the end if lanes took it
+  }
   if (mixed != 0)
     return pressure != nullptr ? reactor_group_cp(n_s, indx_cp_l, indx_cp_r, A, ncu, wg_per_cu, st)
                                : reactor_group_cv(n_s, indx_cp_l, indx_cp_r, A, ncu, wg_per_cu, st);

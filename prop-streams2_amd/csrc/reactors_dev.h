@@ -166,6 +166,12 @@ inline int reactor_grid(int ncu, int wg_per_cu, int min_per_cu, int per_wg, long
 int reactor_ref_cv(int n_s, int indx_cp_l, int indx_cp_r, const ReactorArgs &A, int ncu, int wg_per_cu, hipStream_t st);
 int reactor_ref_cp(int n_s, int indx_cp_l, int indx_cp_r, const ReactorArgs &A, int ncu, int wg_per_cu, hipStream_t st);
 
+// one lane per reactor (reactors_lanes.hip) where a large FP64 species-block batch takes single
+// steps; from as many reactors as fill the GPU at one wave per SIMD
+int reactor_lanes(int n_s, int indx_cp_l, int indx_cp_r, const ReactorArgs &A, int ncu, int wg_per_cu, hipStream_t st);
+constexpr int LANES_FROM = 65536;
+constexpr unsigned LANES_TAKE = 0x80000000u;   // the counter's first value when lanes take the batch
+
 // the species-block forms (reactors_group_dev.h), compiled in reactors_group.hip (constant
 // volume) and reactors_group_cp.hip (constant pressure)
 int reactor_group_cv(int n_s, int indx_cp_l, int indx_cp_r, const ReactorArgs &A, int ncu, int wg_per_cu, hipStream_t st);

@@ -147,11 +147,32 @@ __device__ inline void row_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+constexpr int QMAX = 64;            // reactions whose rates a row keeps at once
+
+// The order in which a row's lanes take the reactions: fall-off forms first, then third-body
+// ones, then the others, so that the lanes of a pass share their branches.  All threads call;
+// the caller synchronises.  More than QMAX reactions are taken in their own order.
+__device__ inline void rate_order(const KinPacked &K, int *order, int *kind) {
+  const int n = K.nr < QMAX ? K.nr : QMAX;
+  if ((int)threadIdx.x < n) {
+    const int ty = ((const int *)(K.pack + KREC * threadIdx.x))[KI_TY];
+    kind[threadIdx.x] = K.nr > QMAX ? 0 : (ty > 2 ? 2 : ty);
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < n) {
+    const int k = kind[threadIdx.x];
+    int rank = 0;
+    for (int q = 0; q < n; ++q) rank += kind[q] > k || (kind[q] == k && q < (int)threadIdx.x) ? 1 : 0;
+    order[rank] = threadIdx.x;
+  }
+}
+
 // chemistry_source_packed of one state with a reaction per lane: c is species l's
-// concentration, the result component l of the source.  The rates of 16 reactions meet in
-// LDS and lane l subtracts them in ascending order.
+// concentration, the result component l of the source.  The rates meet in LDS and lane l
+// subtracts them in ascending order.
 template <int NS>
-__device__ inline double row_source(const KinPacked &K, double tt, double c, double *cl, double *ql, int l) {
+__device__ inline double row_source(const KinPacked &K, double tt, double c, double *cl, double *ql, const int *order,
+                                    int l) {
   const double Rtti = 1.0 / (K.r_univ * tt);
   const double lnT = log(tt);
   int itt = (int)((tt - K.t_min_tab) / K.dt_tab) + 1;
@@ -162,16 +183,16 @@ __device__ inline double row_source(const KinPacked &K, double tt, double c, dou
   const long ntab = (long)K.num_t_tab + 1;
   double acc = 0.0;
   cl[l] = c;
-  for (int r0 = 0; r0 < K.nr; r0 += GROW) {
-    const int r = r0 + l;
+  for (int r0 = 0; r0 < K.nr; r0 += QMAX) {
+    const int n = K.nr - r0 < QMAX ? K.nr - r0 : QMAX;
     row_sync();
-    if (r < K.nr) {
+    for (int i = l; i < n; i += GROW) {
+      const int q = order[i], r = r0 + q;
       const double *R = K.pack + KREC * r;
-      ql[l] = reaction_progress<NS>(R, (const int *)R, K.kc_tab + (itt - 1) + ntab * r, tt, lnT, Rtti, dtt,
+      ql[q] = reaction_progress<NS>(R, (const int *)R, K.kc_tab + (itt - 1) + ntab * r, tt, lnT, Rtti, dtt,
                                     [&](int s) { return cl[s]; }, [&](int s) { return cl[s]; });
     }
     row_sync();
-    const int n = K.nr - r0 < GROW ? K.nr - r0 : GROW;
     const double *net = K.pack + KREC * r0 + KD_NET + l;
 #pragma unroll 4
     for (int k = 0; k < n; ++k) acc = acc - ql[k] * net[KREC * k];
@@ -193,9 +214,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 
   constexpr double e1 = 17.0 / 54.0, e2 = 7.0 / 36.0, e3 = 0.0, e4 = 125.0 / 108.0;
   __shared__ double tlds[thermo_lds_doubles<NS>(WHICH)];
   __shared__ double jbuf[256 / GROW][NS * (GROW + 1)];
-  __shared__ double cbuf[256 / GROW][2 * GROW];
+  __shared__ double cbuf[256 / GROW][GROW + QMAX];
+  __shared__ int order[QMAX], kind[QMAX];
   __shared__ double lane_conc[NS * 256];
+  // taken by reactors_lanes; 16384 rows asking the counter in turn would cost 0.2 ms
+  if (MODE == 2 && !CP && *(volatile unsigned *)A.next >= LANES_TAKE) return;
   const ThermoLds TL = thermo_stage<NS, LO>(A.th, tlds, WHICH);
+  rate_order(A.K, order, kind);
   __syncthreads();
   const int l = threadIdx.x % GROW;
   double *J = jbuf[threadIdx.x / GROW];
@@ -220,7 +245,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 
     static_for<0, NS>([&](auto S) { wv[S] = row_bcast<S>(v); });
     static_for<0, 4>([&](auto S) { wv[NS + S] = mom[S]; });
     rhs_fn().prepare(wv, tg, rho, ri, scale);
-    return -row_source<NS>(A.K, tg, rho * (v * ri) / mwl, cl, ql, l);
+    return -row_source<NS>(A.K, tg, rho * (v * ri) / mwl, cl, ql, order, l);
   };
   // scale * r + x
   auto scaled_plus = [&](double r, double scale, double x) { return CP ? fma(r, scale, x) : r + x; };

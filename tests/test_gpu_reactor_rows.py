@@ -69,3 +69,32 @@ def test_ragged_batches_give_the_same_bits(pkg, mech, pressure, form):
         ref = run(130, 0)[0]
         scale = np.abs(ref[:tb.n_species]).sum(axis=0)
         assert np.max(np.abs(whole[0] - ref)[:tb.n_species] / scale) < 1e-6
+
+
+@pytest.mark.parametrize("mech", ["h2", "keromnes"])
+@pytest.mark.parametrize("first", [1e-9, 1e-7])
+@pytest.mark.parametrize("budget", [0, 1])
+def test_large_fp64_block_batches_give_the_same_bits(pkg, mech, first, budget):
+    """From 65536 constant-volume reactors on, form 2 takes one lane per reactor where the first step
+    spans the interval (first = the horizon), rows elsewhere: the same bits as in small batches,
+    also resumed, with some reactors finished before."""
+    tb = _tables(pkg, mech)
+    be = pkg.solver.HipBackend()
+    R = pkg.reactors.ReactorBatchGPU(be, tb)
+    n, few, horizon = 65536 + 77, 300, 1e-7
+    w0, t0 = _inputs(pkg, tb, 512, False)
+    pick = np.arange(n) % 512
+
+    def run(count):
+        w, tg = be.asarray(np.ascontiguousarray(w0[:, pick[:count]])), be.asarray(t0[pick[:count]])
+        dt, end = be.asarray(np.full(count, first)), be.asarray(np.full(count, horizon))
+        nacc, nrej = be.zeros((count,), "i4"), be.zeros((count,), "i4")
+        td = dn = None
+        if budget:
+            td, dn = be.asarray(np.where(np.arange(count) % 5 == 0, horizon, 0.0)), be.zeros((count,))
+        R.integrate(w, tg, dt, end, nacc, nrej, mixed=2, t_done=td, dt_next=dn, maxsteps=budget or None)
+        return [be.to_numpy(a) for a in (w, tg, nacc, nrej) + ((td, dn) if budget else ())]
+
+    print(f"[lanes] {mech} first {first} budget {budget}", flush=True)
+    for a, b in zip(run(few), run(n)):
+        np.testing.assert_array_equal(a, b[..., :few])
