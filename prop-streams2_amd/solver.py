@@ -534,13 +534,15 @@ class Solver:
         """The substep's right-hand side in one pass over the cells (streams_rhs_cells): a 3-D
         box whose faces all take the KEEP flux of one order (no sensor, no order reduction at
         the boundaries), nkeep = 0, sixth or eighth order throughout, NASA7 tables, and planes
-        within the kernel's 32-bit byte offsets.  Everything else takes the sweeps."""
+        within the kernel's 32-bit byte offsets.  Everything else takes the sweeps, which also
+        refuse a WENO stencil that does not exist or does not fit the ghost layers."""
         n = self.num
         ng = self.ng
         plane = (self.nx + 2 * ng) * (self.ny + 2 * ng) * (self.nz + 2 * ng)
         return (self._full_order and n.sensor_threshold >= 1.0 and n.nkeep == 0 and n.ep_order in (6, 8)
                 and n.visc_order == n.ep_order and min(self.nx, self.ny, self.nz) > 1 and not any(self.force_zero_flux)
-                and self.tb.indx_cp_l == 0 and plane < 1 << 29 and self.be.has("rhs_cells"))
+                and 1 <= n.weno_scheme <= min(4, ng) and self.tb.indx_cp_l == 0 and plane < 1 << 29
+                and self.be.has("rhs_cells"))
 
     def rk_substep_fused(self, istep: int, fold_next: bool = False):
         """One RK substep in five passes: halo + aux, sensor, fused x/y/z sweeps (with
