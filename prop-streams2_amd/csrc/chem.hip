@@ -12,32 +12,40 @@ namespace streams {
 
 // The reference's dense tables are packed into one record per reaction in LDS (kinpack.h) once
 // per workgroup, each of which takes many cells: walking the dense rows costs a uniform branch
-// per species and side of every reaction (0.288 ms for 96x72x60 cells, 9 species and
-// 21 reactions; packed 0.19 ms, bounded by the exponentials and powers of the reference's rate
-// forms, which are kept: folding b ln T into one exponential with -Ea/RT takes another 0.04 ms off
-// but has 1.2 to 1.4 times the error).
-// A mechanism with a side of more than KSIDE species, or with more records than LDS holds
-// (PACKED = false), walks the dense tables.  LO: NASA form of the tables staged in LDS, 99: any
-// other form, from global memory.
+// per species and side of every reaction (96x72x60 cells, 9 species and 21 reactions 0.29 ms dense,
+// 0.17 packed; 14 species and 29 reactions 0.65 and 0.33), bounded by the exponentials and powers of the
+// reference's rate forms, which both walks keep: folding b ln T into one exponential with -Ea/RT takes
+// 0.04 ms off but has 1.2 to 1.4 times the error.
+// PACKED = false walks the dense tables: a mechanism with more records than LDS holds, or with a
+// side of more than KSIDE species, for which both are launched and each looks whether the call is its
+// own (checked; 3 to 9 us in small fields).  In a kernel of its own, because its registers would halve
+// the waves of the packed walk and a loop over cells its own: 160^3 cells, 14 species and 87 reactions
+// 27.4 ms together, 15.0 apart; 9 species with a side of five 2.81 and 2.31.
+// LO: NASA form of the tables staged in LDS, 99: any other form, from global memory.
 template <int NS, int LO, bool PACKED>
 __global__ void __launch_bounds__(256) chemistry_kernel(Box b, double *__restrict__ w, double *__restrict__ w_aux,
                                                         double *__restrict__ fl, Kin K, Thermo th,
-                                                        double tol_iter_nr, unsigned ncells) {
+                                                        double tol_iter_nr, unsigned ncells, bool checked) {
   using X = Idx<NS>;
   constexpr bool STAGED = LO != 99;
   extern __shared__ double rec[];
   __shared__ double tlds[STAGED ? thermo_lds_doubles<NS>(TH_CV | TH_CVH) : 1];
-  __shared__ int dense;
+  __shared__ int flag;
   ThermoLds TL{};
-  if (threadIdx.x == 0) dense = PACKED ? 0 : 1;
-  __syncthreads();
-  if constexpr (STAGED) TL = thermo_stage<NS, LO>(th, tlds, TH_CV | TH_CVH);
-  if constexpr (PACKED)
+  if constexpr (PACKED) {
+    if (threadIdx.x == 0) flag = 1;
+    __syncthreads();
+    if constexpr (STAGED) TL = thermo_stage<NS, LO>(th, tlds, TH_CV | TH_CVH);
     for (int lr = threadIdx.x; lr < K.nr; lr += 256)
-      if (!pack_record(rec + KREC * lr, NS, lr, K.nr, K)) dense = 1;
-  __syncthreads();
-  const bool packed = dense == 0;
+      if (!pack_record(rec + KREC * lr, NS, lr, K.nr, K)) flag = 0;
+    __syncthreads();
+    if (flag == 0) return;
+  } else {
+    if (checked && sides_fit(NS, K, &flag)) return;
+  }
   const long ps = b.pstride(), fs_ = b.fstride(), ntab = (long)K.num_t_tab + 1;
+  // the dense walk takes one cell a thread: about a loop, the constants of its exponentials
+  // would be kept in registers throughout
   for (unsigned t = blockIdx.x * 256u + threadIdx.x; t < ncells; t += gridDim.x * 256u) {
     const long pt = b.p(1 + (int)(t % b.nx), 1 + (int)(t / b.nx % b.ny), 1 + (int)(t / b.nx / b.ny));
     double yy[NS], conc[NS], acc[NS];
@@ -55,7 +63,7 @@ __global__ void __launch_bounds__(256) chemistry_kernel(Box b, double *__restric
       yy[s] = yy[s] * ri;
       w_aux[pt + ps * s] = yy[s];
       conc[s] = rho * yy[s] / K.mw[s];
-      acc[s] = 0.0;
+      acc[s] = PACKED ? 0.0 : fl[t + fs_ * s];
     }
     const double uu = w[pt + ps * (X::I_U - 1)] * ri, vv = w[pt + ps * (X::I_V - 1)] * ri;
     const double ww = w[pt + ps * (X::I_W - 1)] * ri, rhoe = w[pt + ps * (X::I_E - 1)];
@@ -70,42 +78,44 @@ __global__ void __launch_bounds__(256) chemistry_kernel(Box b, double *__restric
       tt = temperature_from_e<NS>(ee, t0, th, tol_iter_nr, yy);
     }
     w_aux[pt + ps * (X::J_T - 1)] = tt;
-    if (packed) {
-      const double Rtti = 1.0 / (K.r_univ * tt);
-      int itt = (int)((tt - K.t_min_tab) / K.dt_tab) + 1;
-      itt = itt < 1 ? 1 : itt;
-      itt = itt > K.num_t_tab ? K.num_t_tab : itt;
-      const double dtt = (tt - ((itt - 1) * K.dt_tab + K.t_min_tab)) / K.dt_tab;
-      for (int lr = 0; lr < K.nr; ++lr) {
+    const double Rtti = 1.0 / (K.r_univ * tt);
+    int itt = (int)((tt - K.t_min_tab) / K.dt_tab) + 1;
+    itt = itt < 1 ? 1 : itt;
+    itt = itt > K.num_t_tab ? K.num_t_tab : itt;
+    const double dtt = (tt - ((itt - 1) * K.dt_tab + K.t_min_tab)) / K.dt_tab;
+    for (int lr = 0; lr < K.nr; ++lr) {
+      if constexpr (PACKED) {
         const double *R = rec + KREC * lr;
         auto c = [&](int s) { return conc[s]; };
         const double q = reaction_progress<NS, true>(R, UniformInts{(const int *)R}, K.kc_tab + (itt - 1) + ntab * lr,
                                                      tt, 0.0, Rtti, dtt, c, c);
 #pragma unroll
         for (int s = 0; s < NS; ++s) acc[s] = acc[s] - q * R[KD_NET + s];
+      } else {
+        const double q = progress_rate<NS>(K, lr, tt, Rtti, itt, dtt, conc);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) acc[s] = acc[s] - (K.p_co[lr + K.nr * s] - K.r_co[lr + K.nr * s]) * q * K.mw[s];
       }
-    } else {
-      chemistry_source<NS>(K, tt, conc, acc);
     }
 #pragma unroll
-    for (int s = 0; s < NS; ++s) fl[t + fs_ * s] = fl[t + fs_ * s] + acc[s];
+    for (int s = 0; s < NS; ++s) fl[t + fs_ * s] = PACKED ? fl[t + fs_ * s] + acc[s] : acc[s];
+    if constexpr (!PACKED) break;
   }
 }
 
-// workgroups of chemistry_kernel: each packs the tables once, so no more than fill the GPU
+// workgroups of the packed walk: each packs the tables once, so no more than fill the GPU
 constexpr long CHEM_BLOCKS = 1024;
 constexpr long CHEM_LDS = 48 * 1024;         // bytes of records at most, beside up to 8 KB of NASA tables
 
 template <int NS, int LO>
 void chemistry_launch(const Box &b, double *w, double *w_aux, double *fl, const Kin &K, const Thermo &th, double tol,
                       unsigned n, hipStream_t st) {
-  long g = ((long)n + 255) / 256;
-  g = g < CHEM_BLOCKS ? g : CHEM_BLOCKS;
-  const long bytes = (long)K.nr * KREC * 8;
-  if (K.nr > 0 && bytes <= CHEM_LDS)
-    chemistry_kernel<NS, LO, true><<<(unsigned)g, 256, bytes, st>>>(b, w, w_aux, fl, K, th, tol, n);
-  else
-    chemistry_kernel<NS, LO, false><<<(unsigned)g, 256, 0, st>>>(b, w, w_aux, fl, K, th, tol, n);
+  const long g = ((long)n + 255) / 256, bytes = (long)K.nr * KREC * 8;
+  const bool packed = K.nr > 0 && bytes <= CHEM_LDS;
+  if (packed)
+    chemistry_kernel<NS, LO, true><<<(unsigned)(g < CHEM_BLOCKS ? g : CHEM_BLOCKS), 256, bytes, st>>>(b, w, w_aux, fl, K,
+                                                                                                     th, tol, n, true);
+  chemistry_kernel<NS, 99, false><<<(unsigned)g, 256, 0, st>>>(b, w, w_aux, fl, K, th, tol, n, packed);
 }
 
 // ------------------------------------------------------------------ Rosenbrock
