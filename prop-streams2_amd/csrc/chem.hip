@@ -218,8 +218,8 @@ extern "C" int streams_rosenbrock(int n_s, int nv, int nv_aux, int nx, int ny, i
   Kin K{mw, arr_a, arr_b, arr_ea, tb_eff, falloff_coeffs, r_coeffs, p_coeffs, kc_tab, reac_ty, isrev,
         nreactions, num_t_tab, t_min_tab, dt_tab, r_univ};
   Thermo th{cv_coeff, nullptr, trange, nsetcv, indx_cp_l, indx_cp_r};
-  const bool rows = (indx_cp_l == 0 || indx_cp_l == -2) && indx_cp_r == 4 && (long)nreactions * KREC * 8 <= ROWS_LDS &&
-                    n <= ROWS_CELLS;
+  const bool rows = (indx_cp_l == 0 || indx_cp_l == -2) && indx_cp_r == 4 && nreactions >= 0 &&
+                    (long)nreactions * KREC * 8 <= ROWS_LDS && n <= ROWS_CELLS;
   hipStream_t st = as_stream(stream);
   if (rows) {
     const int rc = rosenbrock_rows(n_s, b, w, w_aux, K, th, tol_iter_nr, dttry, time_start, time_end, maxsteps,

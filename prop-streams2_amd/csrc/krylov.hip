@@ -287,8 +287,8 @@ extern "C" int streams_rosenbrock_krylov(int n_s, int nv, int nv_aux, int nx, in
         nreactions, num_t_tab, t_min_tab, dt_tab, r_univ};
   Thermo th{cv_coeff, nullptr, trange, nsetcv, indx_cp_l, indx_cp_r};
   const double *fls = simpler_splitting == 1 ? fl_sav : nullptr;
-  const bool rows = (indx_cp_l == 0 || indx_cp_l == -2) && indx_cp_r == 4 && (long)nreactions * KREC * 8 <= KROWS_LDS &&
-                    n <= KROWS_CELLS;
+  const bool rows = (indx_cp_l == 0 || indx_cp_l == -2) && indx_cp_r == 4 && nreactions >= 0 &&
+                    (long)nreactions * KREC * 8 <= KROWS_LDS && n <= KROWS_CELLS;
   hipStream_t st = as_stream(stream);
   if (rows) {
     const int rc = krylov_rows(n_s, b, w, w_aux, K, th, tol_iter_nr, dttry, time_start, time_end, maxsteps, fls, pasr, st);
