@@ -10,7 +10,7 @@
 //     chain, then run in turn on those sums in every lane; the 16 reaction sources run side by side;
 //   * momentum and energy have no source: their Jacobian rows are zero and their stages are zero,
 //     so the solves are those of the species block.  Their columns only enter the row maxima of
-//     the implicit pivoting.
+//     the implicit pivoting, and where one is not finite no component is.
 // One lane per cell kept the Jacobian, its factors and the stages in 4.5 to 7 KB of scratch and
 // walked 2 (N_S + 4) + 1 right-hand sides one after the other.  Measured, one lane -> a row, same
 // bits: 60 constant-pressure reactors of 9 species, 12 steps 65 -> 3.4 ms, of 14 species, 8 steps
@@ -332,10 +332,19 @@ __global__ void __launch_bounds__(REF_BS) __attribute__((amdgpu_waves_per_eu(2))
       const double j = jrow[C * JS];
       a[C] = l == C ? gi - j : -j;
     });
-    static_for<NS, NV>([&](auto C) { amax = fabs(jrow[C * JS]) > amax ? fabs(jrow[C * JS]) : amax; });
+    bool bad = false;
+    static_for<NS, NV>([&](auto C) {
+      const double j = fabs(jrow[C * JS]);
+      amax = j > amax ? j : amax;
+      bad = bad || !(j < HUGE_VAL);
+    });
     int perm;
     row_ludcmp<NS, double>(a, l, perm, amax);
-    const double g1 = row_solve<NS>(jrow, a, l, perm, gi, rhs_sav);
+    // a non-finite entry of those columns makes the momentum and energy pivots, and through their
+    // stages every component, not a number
+    const bool lost = ((__ballot(l < NS && bad) >> (threadIdx.x & 48)) & 0xffff) != 0;
+    double g1 = row_solve<NS>(jrow, a, l, perm, gi, rhs_sav);
+    if (lost) g1 = __builtin_nan("");
     time = t0 + dt;
     double scale;
     double rhs = rhs_stage(fma(a21, g1, wsav), scale);
