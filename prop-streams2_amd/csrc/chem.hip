@@ -122,11 +122,13 @@ void chemistry_launch(const Box &b, double *w, double *w_aux, double *fl, const 
 int rosenbrock_rows(int n_s, const Box &b, double *w, double *w_aux, const Kin &K, const Thermo &th,
                     double tol_iter_nr, double dttry, double time_start, double time_end, int maxsteps, int maxtry,
                     double tol, const Pasr &pasr, hipStream_t st);
-// Cells above which one lane per cell fills the GPU (256 CUs x 2 waves per SIMD), and the idle
-// lanes of a row's Newton chain cost more than the scratch of a lane's Jacobian: random states, one
-// interval of 2 ns, 28800 cells of 9 species 67.7 -> 33.0 ms, 115200 cells of 14 species 450 ->
-// 378, but 414720 cells of 9 species 320 -> 398.
-constexpr long ROWS_CELLS = 131072;
+// Cells up to which rows are no slower where every cell takes one step: the time of the rows grows with the
+// cells, that of one lane per cell only once the GPU is full.  One lane -> rows, ms: 9 species 24576
+// cells 2.62 -> 1.71, 40960 3.15 -> 2.77, 65536 3.41 -> 4.40; 13 species 24576 7.03 -> 6.47, 26624 7.08 ->
+// 7.12, 32768 7.30 -> 8.61; 14 species 26624 8.63 -> 7.45, 32768 8.92 -> 9.06, 131072 14.1 -> 35.9.  Where cells
+// differ in their steps rows win far beyond (random radical pools, 14 species, 65536 cells 1050 -> 420),
+// which the call cannot know.
+inline long rows_cells(int n_s) { return n_s <= 9 ? 40960 : 26624; }
 constexpr long ROWS_LDS = 36 * 1024;         // bytes of records at most, beside the rows' own 24 KB
 
 // 2 waves per SIMD (the compiler's own choice is 1, with 2.8-3.7 KB of per-lane spills):
@@ -219,7 +221,7 @@ extern "C" int streams_rosenbrock(int n_s, int nv, int nv_aux, int nx, int ny, i
         nreactions, num_t_tab, t_min_tab, dt_tab, r_univ};
   Thermo th{cv_coeff, nullptr, trange, nsetcv, indx_cp_l, indx_cp_r};
   const bool rows = (indx_cp_l == 0 || indx_cp_l == -2) && indx_cp_r == 4 && nreactions >= 0 &&
-                    (long)nreactions * KREC * 8 <= ROWS_LDS && n <= ROWS_CELLS;
+                    (long)nreactions * KREC * 8 <= ROWS_LDS && n <= rows_cells(n_s);
   hipStream_t st = as_stream(stream);
   if (rows) {
     const int rc = rosenbrock_rows(n_s, b, w, w_aux, K, th, tol_iter_nr, dttry, time_start, time_end, maxsteps,
