@@ -253,10 +253,13 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) k
 int krylov_rows(int n_s, const Box &b, double *w, const double *w_aux, const Kin &K, const Thermo &th,
                 double tol_iter_nr, double dttry, double time_start, double time_end, int maxsteps,
                 const double *fl_sav, const Pasr &pasr, hipStream_t st);
-// Cells up to which half a wave per cell is faster (random states, one interval of 1e-8 s, 9
-// species): 800 cells 939 -> 236 ms, 8000 cells 1079 -> 774; 4096 cells are in flight at once, above
-// some 8000 the repeated scalar work of the 32 lanes costs what the shorter chain gains.
-constexpr long KROWS_CELLS = 8192;
+// Cells up to which half a wave per cell is faster where every cell takes the same steps: 4096 cells are
+// in flight at once, and beyond them the time grows with the cells, while that of one lane per cell
+// stays as it is until the GPU is full.  One lane -> rows, us (an interval of 1e-8 s): 9 species 4096
+// cells 842 -> 562, 6144 835 -> 646, 8192 827 -> 1078; 14 species 4096 1700 -> 842, 8192 1844 -> 1610,
+// 16384 1895 -> 3179; 13 species 8192 1621 -> 1581.  Where cells differ in their steps rows win further out
+// (random radical pools, 9 species, 8000 cells 1079 -> 774 ms), which the call cannot know.
+inline long krows_cells(int n_s) { return n_s <= 9 ? 6144 : 8192; }
 constexpr long KROWS_LDS = 36 * 1024;        // bytes of records at most
 
 }  // namespace streams
@@ -288,7 +291,7 @@ extern "C" int streams_rosenbrock_krylov(int n_s, int nv, int nv_aux, int nx, in
   Thermo th{cv_coeff, nullptr, trange, nsetcv, indx_cp_l, indx_cp_r};
   const double *fls = simpler_splitting == 1 ? fl_sav : nullptr;
   const bool rows = (indx_cp_l == 0 || indx_cp_l == -2) && indx_cp_r == 4 && nreactions >= 0 &&
-                    (long)nreactions * KREC * 8 <= KROWS_LDS && n <= KROWS_CELLS;
+                    (long)nreactions * KREC * 8 <= KROWS_LDS && n <= krows_cells(n_s);
   hipStream_t st = as_stream(stream);
   if (rows) {
     const int rc = krylov_rows(n_s, b, w, w_aux, K, th, tol_iter_nr, dttry, time_start, time_end, maxsteps, fls, pasr, st);
