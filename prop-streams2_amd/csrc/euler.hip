@@ -219,7 +219,7 @@ __global__ void __launch_bounds__(128) euler_yz_fused_kernel(Box b, EulerArgs A,
 // 0.40 -> 0.062, z 0.40 -> 0.077).  Bounded by the loads of the L1: 16 clocks of a CU per wave's
 // load, seven cells of each variable.  Any order takes this form: the loads of the levels above
 // lmax are skipped.  Cells beside an order-reduced or zeroed face
-// are left to euler_edge_kernel.  nkeep <= 0.
+// are left to euler_edges.  nkeep <= 0.
 template <int DIR>
 __device__ inline bool cell_of_sweep(const Box &b, const EulerArgs &A, unsigned t, int &t1, int &t2, int &c) {
   // x: the cell fastest; y, z: i fastest, then the other index, then the cell
@@ -246,11 +246,11 @@ __device__ inline int cell_order(const Box &b, const EulerArgs &A, int t1, int t
 }
 
 template <int NS, int DIR>
-__global__ void __launch_bounds__(256) euler_cell_kernel(Box b, EulerArgs A) {
+__device__ inline void euler_cell(const Box &b, const EulerArgs &A, unsigned block) {
   using X = Idx<NS>;
   constexpr int LB = 4;
   int t1, t2, c;
-  if (!cell_of_sweep<DIR>(b, A, blockIdx.x * 256u + threadIdx.x, t1, t2, c)) return;
+  if (!cell_of_sweep<DIR>(b, A, block * 256u + threadIdx.x, t1, t2, c)) return;
   const int lmax = cell_order<DIR>(b, A, t1, t2, c);
   if (lmax == 0) return;
   Line L{A.w_aux, 0, 0, b.pstride()};
@@ -305,16 +305,13 @@ __global__ void __launch_bounds__(256) euler_cell_kernel(Box b, EulerArgs A) {
   }
 }
 
-// The cells euler_cell_kernel leaves: both face fluxes in full, each at its own order; a
+// A cell that euler_cell leaves: both face fluxes in full, each at its own order; a
 // zeroed face keeps its pressure alone.  Every pair of the highest order is an unrolled, predicated term, so lanes of
 // different order share one instruction stream.
 template <int NS, int DIR>
-__global__ void __launch_bounds__(256) euler_edge_kernel(Box b, EulerArgs A) {
+__device__ inline void euler_edge_cell(const Box &b, const EulerArgs &A, int t1, int t2, int c) {
   using X = Idx<NS>;
   constexpr int LB = 4, NP = LB * (LB + 1) / 2;
-  int t1, t2, c;
-  if (!cell_of_sweep<DIR>(b, A, blockIdx.x * 256u + threadIdx.x, t1, t2, c)) return;
-  if (cell_order<DIR>(b, A, t1, t2, c) != 0) return;
   Line L{A.w_aux, 0, 0, b.pstride()};
   line_base<DIR>(b, t1, t2, L.base, L.st);
   const double met = A.metric[c - 1];
@@ -384,6 +381,48 @@ __global__ void __launch_bounds__(256) euler_edge_kernel(Box b, EulerArgs A) {
   }
 }
 
+// A workgroup lists the cells left among 256 * PER and spreads them over its threads: along x they
+// are the ends of every row, a few lanes of nearly every wave (96x72x60 cells, sixth order, walls at both
+// ends of x: both kernels 125 -> 79 us).
+template <int NS, int DIR, int PER>
+__device__ inline void euler_edges(const Box &b, const EulerArgs &A, unsigned block) {
+  __shared__ unsigned list[256 * PER], count;
+  if (threadIdx.x == 0) count = 0;
+  __syncthreads();
+  int t1, t2, c;
+  for (unsigned q = 0; q < PER; ++q) {
+    const unsigned t = (block * PER + q) * 256u + threadIdx.x;
+    if (cell_of_sweep<DIR>(b, A, t, t1, t2, c) && cell_order<DIR>(b, A, t1, t2, c) == 0) list[atomicAdd(&count, 1u)] = t;
+  }
+  __syncthreads();
+  for (unsigned q = threadIdx.x; q < count; q += 256u) {
+    cell_of_sweep<DIR>(b, A, list[q], t1, t2, c);
+    euler_edge_cell<NS, DIR>(b, A, t1, t2, c);
+  }
+}
+
+// along y and z the cells left are whole rows, which fill their waves as they are
+template <int DIR>
+constexpr int edge_per() { return DIR == 1 ? 4 : 1; }
+template <int NS, int DIR>
+__global__ void __launch_bounds__(256) euler_cell_kernel(Box b, EulerArgs A) {
+  euler_cell<NS, DIR>(b, A, blockIdx.x);
+}
+template <int NS, int DIR>
+__global__ void __launch_bounds__(256) euler_edge_kernel(Box b, EulerArgs A) {
+  euler_edges<NS, DIR, edge_per<DIR>()>(b, A, blockIdx.x);
+}
+// Both side by side in one launch, for fields of so few workgroups that the edges' registers (three
+// workgroups a CU) do not limit the cells: 19x14x11 cells with walls, x 38 -> 23 us, y 36 -> 22; but
+// 64x64x64 periodic 41 -> 55.
+constexpr unsigned EULER_ONE = 768;
+template <int NS, int DIR>
+__global__ void __launch_bounds__(256) euler_both_kernel(Box b, EulerArgs A) {
+  const unsigned g = gridDim.x / 2;
+  if (blockIdx.x < g) euler_cell<NS, DIR>(b, A, blockIdx.x);
+  else euler_edges<NS, DIR, 1>(b, A, blockIdx.x - g);
+}
+
 template <int NS, int DIR>
 inline int prepass_launch(const Box &b, const EulerArgs &A, int t1n, long nfaces, hipStream_t st) {
   if (nfaces > (long)0xFFFFFF00u) return STREAMS_E_DIMS;
@@ -430,8 +469,12 @@ int euler_launch(const Box &b, EulerArgs A, hipStream_t st) {
     if (rc) return rc;
   } else if (A.nkeep <= 0 && (long)(nf - 1) * t1n * t2n < 0xffffff00l) {
     const unsigned g = blocks_for((long)(nf - 1) * t1n * t2n, 256);
-    euler_cell_kernel<NS, DIR><<<g, 256, 0, st>>>(b, A);
-    euler_edge_kernel<NS, DIR><<<g, 256, 0, st>>>(b, A);
+    if (g <= EULER_ONE) {
+      euler_both_kernel<NS, DIR><<<2 * g, 256, 0, st>>>(b, A);
+    } else {
+      euler_cell_kernel<NS, DIR><<<g, 256, 0, st>>>(b, A);
+      euler_edge_kernel<NS, DIR><<<(g + edge_per<DIR>() - 1) / edge_per<DIR>(), 256, 0, st>>>(b, A);
+    }
     return hip_status();
   }
   if (DIR == 1) {
