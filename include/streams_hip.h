@@ -473,7 +473,10 @@ int streams_rhs_cells(int n_s, int nx, int ny, int nz, int ng, int nv_aux, int l
  * reached (time_end[b] when done) and the step it would take next.  Kinetics come from the device copy of
  * streams_kinetics_pack.  work is one unsigned of device memory for the shared work
  * counter (zeroed by the call on the stream); wg_per_cu workgroups of 256 lanes per CU form
- * the persistent grid (4 when wg_per_cu <= 0; never more than the batch needs).
+ * the persistent grid (4 when wg_per_cu <= 0; never more than the batch needs).  Batches of
+ * mixed = 1 and 2 from 12288 reactors on (40960 beyond 9 species) may take 28 bytes a reactor of
+ * stream-ordered memory (hipMallocAsync) for the call; recorded in a graph, or where there is none,
+ * they do without.
  * mixed = 0 is the plain FP64 integrator in the reference's arithmetic forms (central-
  * difference Jacobian over all N_S + 4 variables, FP64 LU, rosenbrock_rhs's forms of the
  * rate expressions and of the temperature inversion): the yardstick of the other forms.

@@ -123,6 +123,15 @@ struct RosRhsPressure {
   }
 };
 
+// Reactors that the lanes leave to the rows: r's time, next step (finish: it ends the interval) and
+// steps so far, at its own place; the list of them, and two counters (how many, and how many
+// the rows have taken).  n null: the lanes integrate every reactor to its end.
+struct LaneLeft {
+  unsigned *n, *list;
+  double *time, *dt;
+  int *nacc, *nrej2;              // accepted; 2 * rejected + finish
+};
+
 struct ReactorArgs {
   double *w, *tg;                 // w[m * nbatch + b] (SoA), T guess / result
   const double *dttry, *time_end; // per reactor
@@ -135,6 +144,7 @@ struct ReactorArgs {
   const double *pressure;         // per reactor; null: constant volume
   KinPacked K;
   Thermo th;
+  LaneLeft left;
 };
 
 // Persistent grid: wg_per_cu workgroups per CU (default 4, at least the resident capacity
@@ -166,10 +176,16 @@ inline int reactor_grid(int ncu, int wg_per_cu, int min_per_cu, int per_wg, long
 int reactor_ref_cv(int n_s, int indx_cp_l, int indx_cp_r, const ReactorArgs &A, int ncu, int wg_per_cu, hipStream_t st);
 int reactor_ref_cp(int n_s, int indx_cp_l, int indx_cp_r, const ReactorArgs &A, int ncu, int wg_per_cu, hipStream_t st);
 
-// one lane per reactor (reactors_lanes.hip) where a large FP64 species-block batch takes single
-// steps; from as many reactors as fill the GPU at one wave per SIMD
-int reactor_lanes(int n_s, int indx_cp_l, int indx_cp_r, const ReactorArgs &A, int ncu, int wg_per_cu, hipStream_t st);
-constexpr int LANES_FROM = 65536;
+// one lane per reactor (reactors_lanes_dev.h): form 2, and form 1 up to LANES_NS species
+int reactor_lanes_cv(int n_s, int indx_cp_l, int indx_cp_r, const ReactorArgs &A, int ncu, int wg_per_cu, hipStream_t st);
+int reactor_lanes_cp(int n_s, int indx_cp_l, int indx_cp_r, const ReactorArgs &A, int ncu, int wg_per_cu, hipStream_t st);
+int reactor_lanes_cv_wide(int n_s, int indx_cp_l, int indx_cp_r, const ReactorArgs &A, int ncu, int wg_per_cu,
+                          hipStream_t st);
+int reactor_lanes_cp_wide(int n_s, int indx_cp_l, int indx_cp_r, const ReactorArgs &A, int ncu, int wg_per_cu,
+                          hipStream_t st);
+constexpr int LANES_NS = 9;
+constexpr int LANE_STEPS = 24;                 // steps that the lanes take where they may leave a reactor
+constexpr int LANES_NARROW = 65536;            // reactors that the GPU holds at one wave per SIMD
 constexpr unsigned LANES_TAKE = 0x80000000u;   // the counter's first value when lanes take the batch
 
 // the species-block forms (reactors_group_dev.h), compiled in reactors_group.hip (constant

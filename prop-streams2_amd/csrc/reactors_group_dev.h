@@ -217,8 +217,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 
   __shared__ double cbuf[256 / GROW][GROW + QMAX];
   __shared__ int order[QMAX], kind[QMAX];
   __shared__ double lane_conc[NS * 256];
-  // taken by reactors_lanes; 16384 rows asking the counter in turn would cost 0.2 ms
-  if (MODE == 2 && !CP && *(volatile unsigned *)A.next >= LANES_TAKE) return;
+  // What the lanes took is theirs but for the reactors they left.  Read before any row asks the
+  // counter in its turn: 16384 rows asking would cost 0.2 ms.
+  long nb_rows = A.nbatch;
+  bool rest = false;
+  if ((MODE == 2 || NS <= LANES_NS) && *(volatile unsigned *)A.next >= LANES_TAKE) {
+    rest = true;
+    nb_rows = A.left.n ? *(volatile unsigned *)A.left.n : 0;
+    if ((long)blockIdx.x * (256 / GROW) >= nb_rows) return;
+  }
+  unsigned *const counter = rest ? A.left.n + 1 : A.next;
   const ThermoLds TL = thermo_stage<NS, LO>(A.th, tlds, WHICH);
   rate_order(A.K, order, kind);
   __syncthreads();
@@ -252,9 +260,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 
   for (;;) {
     if (!active) {
       unsigned q = 0;
-      if (l == 0) q = atomicAdd(A.next, 1u);
+      if (l == 0) q = atomicAdd(counter, 1u);
       r = (unsigned)row_bcast<0>((int)q);
-      if ((long)r >= nb) break;
+      if ((long)r >= nb_rows) break;
+      if (rest) r = A.left.list[r];
       if (l < NS) w = A.w[(long)l * nb + r];
       static_for<0, 4>([&](auto S) { mom[S] = A.w[(long)(NS + S) * nb + r]; });
       tg = A.tg[r];
@@ -265,7 +274,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 
       nacc = nrej = finish = 0;
       iter = 1;
       fresh = active = true;
-      if (A.t_done) {
+      if (rest) {
+        time = A.left.time[r];
+        dt = A.left.dt[r];
+        nacc = A.left.nacc[r];
+        nrej = A.left.nrej2[r] >> 1;
+        finish = A.left.nrej2[r] & 1;
+        iter = nacc + 1;
+      } else if (A.t_done) {
         time = A.t_done[r];
         if (A.dt_next[r] > 0.0) dt = A.dt_next[r];
         if (time >= time_end) {                      // finished earlier: nothing to do
