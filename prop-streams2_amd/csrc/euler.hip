@@ -9,7 +9,8 @@
 //      faces in a typical shear layer but touch a third of the 64-face waves, so the
 //      list keeps the WENO lanes full instead of idling 60 % of each active wave;
 //   2. without the sensor (threshold 1 or more) and nkeep <= 0: a thread per cell and the
-//      telescoped KEEP difference (euler_cell_kernel);
+//      telescoped KEEP difference (euler_cell), and both faces in full for the cells beside
+//      order-reduced or zeroed faces (euler_edges);
 //   3. else a fused pass: every face's KEEP split-form flux (or the parked WENO flux) and
 //      the flux-difference update of fl in the same kernel, so face fluxes never round-
 //      trip through HBM:

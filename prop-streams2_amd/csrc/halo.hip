@@ -3,9 +3,9 @@
 // The reference exchanges ng-deep face slabs through pack -> MPI (or a device copy when
 // the neighbour is the rank itself) -> unpack (base_gpu.F90:1132-1264).  On one GPU the
 // periodic exchange is a direct copy from the opposite interior slab into the ghost slab,
-// one kernel per axis with the two sides and all variables in one grid.  When an axis is
-// shorter than ng the source slab overlaps the ghost slab of the same axis; that case is
-// staged through a device buffer so that every source is read before any ghost is written.
+// one launch for all axes, sides and variables.  When an axis is shorter than ng the source slab
+// overlaps the ghost slab of the same axis; there a thread takes a whole line across both and reads its
+// sources before it writes any of them.  Extrapolation fills any run of faces in one launch as well.
 
 #include "common.h"
 

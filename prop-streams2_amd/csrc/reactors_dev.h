@@ -1,6 +1,6 @@
 // reactors_dev.h — device code of the batched reactor integrator (streams_reactor_batch):
 // arguments, right-hand sides of the species-block forms and the persistent grid.  Included by
-// reactors.hip (the entry point) and reactors_group_dev.h (the kernels).
+// reactors.hip (the entry point), reactors_group_dev.h and reactors_lanes_dev.h (the kernels).
 #pragma once
 #include <type_traits>
 

@@ -1,18 +1,19 @@
 // reactors_group_dev.h — the species-block Rosenbrock integrator of the reactor batch with a
 // 16-lane row of a wave per reactor.
 //
-// Same method and the same operations in the same order as rosenbrock_cell_mp
-// (the ROS4 cell with a one-sided species Jacobian), laid out across lanes:
+// Same method and the same operations in the same order as rosenbrock_cell_block
+// (reactors_lanes_dev.h: the ROS4 cell with a one-sided species Jacobian), laid out across lanes:
 //   * lane n evaluates the right-hand side perturbed in species n, lane NS the unperturbed
 //     one, so a step's N_S + 1 right-hand sides run side by side;
 //   * lane m holds component m of every vector (state, stages) and row m of the matrix, so
-//     nothing is indexed dynamically and nothing spills: one lane per reactor kept the
-//     Jacobian, its factors and the stages in 1.8-4.5 KB of scratch per lane, whose traffic
-//     bounded it (FP64 units 5-8 % busy);
+//     nothing is indexed dynamically and little spills (0.3-0.4 KB a lane): one lane per reactor
+//     keeps the Jacobian, its factors and the stages in 1.2-4.5 KB of scratch per lane, whose
+//     traffic bounds it (FP64 units 5-8 % busy);
 //   * a component reaches the other lanes by row_newbcast DPP moves; the Jacobian is
 //     transposed from columns to rows through LDS, where it stays for a retry of the step.
 // Each row takes its next reactor from the work counter as soon as its own is done: the loop
-// is over step attempts, so a wave waits for no reactor of another row.
+// is over step attempts, so a wave waits for no reactor of another row.  Where lanes began the batch,
+// the rows take the reactors that they left, from the step they had reached.
 #pragma once
 #include "reactors_dev.h"
 
