@@ -7,7 +7,7 @@ import oracle_backend
 
 
 class _Cells(oracle_backend.OracleBackend):
-    """The checker's backend with the fused entry points listed."""
+    """The oracle's backend with the fused entry points listed."""
 
     def has(self, name):
         return True
